@@ -73,6 +73,17 @@ __host__ __device__ __forceinline__ int64_t asm_index4(int row, int col, int ks)
 // whole groups of four fragments without bounds tests.
 __host__ __device__ __forceinline__ int asm_ksteps(int nbt) { return (((nbt + 3) >> 2) + 3) & ~3; }
 
+// Integer division of x < 2^24 by a wave-uniform d via the float reciprocal
+// (exact after one correction step).
+__device__ __forceinline__ int fdiv(int x, int d, float rd)
+{
+  int q = (int)((float)x * rd);
+  int r = x - q * d;
+  if (r < 0) --q;
+  else if (r >= d) ++q;
+  return q;
+}
+
 // One contraction step inside a slab: out[i1 + n1*(q + nout*i3)] =
 // sum_k M[q + nout*k] in[i1 + n1*(k + nin*i3)], M at pool offset `mat`.
 struct StepDev {

@@ -14,6 +14,7 @@
 
 #include "../../include/evr_hip.h"
 #include "evr_internal.hpp"
+#include "evr_hterm.hpp"
 #include "evr_kernels.hpp"
 #include "evr_setup.hpp"
 #include "evr_term.hip"
@@ -83,9 +84,22 @@ struct KClass {
 constexpr KClass kClasses[] = {{256, 1, 4},  {512, 1, 4},  {512, 2, 4}, {512, 2, 2},
                                {512, 4, 2}, {512, 4, 1}, {1024, 4, 1}, {1024, 8, 1}};
 constexpr int kNumClasses = sizeof(kClasses) / sizeof(kClasses[0]);
+// profiling slots: the term classes, the assembled apply, the register-block terms
+constexpr int kProfAsm = kNumClasses, kProfHt = kNumClasses + 1, kProfSlots = kNumClasses + 2;
 // dynamic LDS per workgroup: 160 KiB less a reserve for the kernels' static
 // arrays (about 2 KiB for the term kernels)
 constexpr size_t kLdsLimit = 160 * 1024 - 4096;
+// classes of k_hterm workgroups: vectors per workgroup (1 << lv), LDS bytes at
+// most and threads.  The kernel is built for 16 waves per CU; a class takes
+// the LDS of 1, 2, 3 or 4 workgroups per CU and as many threads as fill them.
+// A term goes to the last class that holds it.
+struct HtClass {
+  int lv, lds, nt;
+};
+constexpr int kKiB = 1024;
+constexpr HtClass kHtClasses[] = {{0, 160 * kKiB, 1024}, {0, 80 * kKiB, 512}, {0, 53 * kKiB, 320}, {0, 40 * kKiB, 256},
+                                  {1, 40 * kKiB, 256},   {2, 40 * kKiB, 256}, {3, 40 * kKiB, 256}};
+constexpr int kHtCaps = sizeof(kHtClasses) / sizeof(kHtClasses[0]);
 // a one-term plan of at least this many functions runs its term streamed
 constexpr int kStreamOneMin = 256;
 
@@ -163,6 +177,20 @@ struct evr_plan {
   std::vector<int> tclass;  // kernel class of every term (static rule or autotuned)
   bool keo_layout = false;  // the term layouts hold the KEO factors in LDS
   size_t lds_bytes64[kNumClasses] = {}, lds_bytes32[kNumClasses] = {};
+  // FP64 H|psi> terms in register blocks (evr_hterm.hip): term and group
+  // records, the matrix, factor and coefficient pools, and the work list
+  // sorted by class (ht_off; ht_lds[c][lv]: LDS bytes of a workgroup of class
+  // c for 1 << lv vectors, ht_items[c]: most pencils of a term).  ht_rest[c]:
+  // terms that stay with the term kernel of class c.
+  bool ht = false, ht_hasM = false;
+  std::vector<char> ht_on;  // per term: runs in register blocks
+  DevBuf<evr::HTerm> d_ht;
+  DevBuf<evr::HGroup> d_hg;
+  DevBuf<double> d_hpool, d_hfac, d_hcoef;
+  DevBuf<int> d_horder, d_ht_rest[kNumClasses];
+  int64_t ht_off[kHtCaps + 1] = {}, ht_nrest[kNumClasses] = {};
+  size_t ht_lds[kHtCaps][4] = {};
+  int ht_items[kHtCaps] = {};
   // work buffers
   DevBuf<double> d_X, d_R, d_psi, d_hpsi, d_G;
   DevBuf<double> d_gw;  // w_t * quadrature weight of every term-grid point (lazy)
@@ -177,12 +205,13 @@ struct evr_plan {
   bool V32_valid = false;
   // per-launch accounting: algorithmic flops per vector of each kernel class
   double flops_class[kNumClasses] = {};
+  double flops_ht = 0, flops_rest[kNumClasses] = {};  // of the register-block terms, of the others
   double flops_reduce = 0;
   bool profiling = false;
-  hipEvent_t ev[2 * (kNumClasses + 1)] = {};
-  double ms_acc[kNumClasses + 1] = {};
-  double flops_acc[kNumClasses + 1] = {};
-  int64_t launches[kNumClasses + 1] = {};
+  hipEvent_t ev[2 * kProfSlots] = {};
+  double ms_acc[kProfSlots] = {};
+  double flops_acc[kProfSlots] = {};
+  int64_t launches[kProfSlots] = {};
 
   evr_plan() = default;
   evr_plan(const evr_plan &) = delete;
@@ -200,6 +229,8 @@ struct evr_plan {
     d_A64.release(); d_A32.release(); d_asm_items.release(); d_D1.release(); d_D2.release();
     d_GG.release(); d_Jg.release(); d_Sg.release(); d_Gg.release(); d_Pg.release(); d_Fg.release();
     d_F2g.release(); d_F1g.release(); d_gitems.release(); d_dp_perm.release(); d_big.release();
+    d_ht.release(); d_hg.release(); d_hpool.release(); d_hfac.release(); d_hcoef.release(); d_horder.release();
+    for (int c = 0; c < kNumClasses; ++c) d_ht_rest[c].release();
     d_Wq.release(); d_As.release(); d_R2.release(); d_F2w.release(); d_F1w.release();
     for (auto &e : ev)
       if (e) (void)hipEventDestroy(e);
@@ -596,6 +627,487 @@ int run_streamed(evr_plan *p, const std::vector<int64_t> &list, int mode, int nv
   return EVR_OK;
 }
 
+// Host inputs of the register-block H|psi> tables: the slots' matrices and
+// factors, and the KEO coefficients by mode.
+struct HtInput {
+  const std::vector<double> &bw, &keo;
+  const std::vector<double> &cC, &cA, &cF1;    // c_ij, a_ijk, F1_i by mode (empty: none)
+  const std::vector<std::vector<int>> &sets;   // position -> mode of every coefficient set
+  int D;                                       // modes of the coefficients
+  int nlev;                                    // slots per mode
+};
+
+// eigenvectors U (columns) and eigenvalues of the symmetric n x n matrix A by
+// cyclic Jacobi rotations
+void jacobi_eig(int n, std::vector<long double> A, std::vector<long double> &U, std::vector<long double> &lam)
+{
+  U.assign((size_t)n * n, 0.0L);
+  for (int i = 0; i < n; ++i) U[i + (size_t)n * i] = 1.0L;
+  for (int sweep = 0; sweep < 60; ++sweep) {
+    long double off = 0.0L, all = 0.0L;
+    for (int i = 0; i < n; ++i)
+      for (int j = 0; j < n; ++j) {
+        const long double v = A[i + (size_t)n * j] * A[i + (size_t)n * j];
+        all += v;
+        if (i != j) off += v;
+      }
+    if (off <= 1e-38L * all) break;
+    for (int p = 0; p < n; ++p)
+      for (int q = p + 1; q < n; ++q) {
+        const long double apq = A[p + (size_t)n * q];
+        if (apq == 0.0L) continue;
+        const long double th = (A[q + (size_t)n * q] - A[p + (size_t)n * p]) / (2.0L * apq);
+        const long double t = (th >= 0 ? 1.0L : -1.0L) / (std::fabs(th) + std::sqrt(th * th + 1.0L));
+        const long double c = 1.0L / std::sqrt(t * t + 1.0L), s = t * c;
+        for (int k = 0; k < n; ++k) {
+          const long double x = A[k + (size_t)n * p], y = A[k + (size_t)n * q];
+          A[k + (size_t)n * p] = c * x - s * y;
+          A[k + (size_t)n * q] = s * x + c * y;
+        }
+        for (int k = 0; k < n; ++k) {
+          const long double x = A[p + (size_t)n * k], y = A[q + (size_t)n * k];
+          A[p + (size_t)n * k] = c * x - s * y;
+          A[q + (size_t)n * k] = s * x + c * y;
+        }
+        for (int k = 0; k < n; ++k) {
+          const long double x = U[k + (size_t)n * p], y = U[k + (size_t)n * q];
+          U[k + (size_t)n * p] = c * x - s * y;
+          U[k + (size_t)n * q] = s * x + c * y;
+        }
+      }
+  }
+  lam.resize(n);
+  for (int i = 0; i < n; ++i) lam[i] = A[i + (size_t)n * i];
+}
+
+// kind of a group of one (nb1 = nq1 = 1) or two modes, kHgGeneric if none
+int hgroup_kind(int nb0, int nq0, int nb1, int nq1)
+{
+#define EVR_K(K, B1, N1, B2, N2) if (nb0 == B1 && nq0 == N1 && nb1 == B2 && nq1 == N2) return K;
+  EVR_HG_KINDS(EVR_K)
+#undef EVR_K
+  return evr::kHgGeneric;
+}
+
+// Tables of the register-block H|psi> (evr_hterm.hip) for the terms that fit
+// a workgroup; with a q-linear G it needs symmetric coordinate matrices W x B
+// (W = B^T diag(w)) and a_iji = a_jii (G symmetric in i, j); other plans keep
+// the term kernels (p->ht stays false).
+int build_hterms(evr_plan *p, const HtInput &h)
+{
+  const int D = p->D, Dm = h.D, ns = (int)p->slots.size();
+  const bool hasA = p->hasA;
+  auto A = [&](int i, int j, int k) { return h.cA[((size_t)i * Dm + j) * Dm + k]; };
+  if (hasA) {
+    double amax = 0.0;
+    for (double v : h.cA) amax = std::max(amax, std::fabs(v));
+    for (int i = 0; i < Dm; ++i)
+      for (int j = 0; j < Dm; ++j)
+        if (std::fabs(A(j, i, j) - A(i, j, j)) > 4e-16 * amax) return EVR_OK;
+  }
+  // ---- per slot: B, W (rotated with a q-linear G) and the rotations, row by
+  // row (a thread's scalar loads take whole rows), and the factor rows
+  // [row][col]{P, T, a_jjj U, R + S} followed by xi
+  std::vector<double> pool, fac;
+  std::vector<int> oB(ns), oW(ns), oI(ns), oO(ns), oF(ns);
+  const int kTd = p->diagT2 ? evr::kT2 : evr::kT;
+  for (int s = 0; s < ns; ++s) {
+    const evr::SlotDev &sd = p->slots[s];
+    const int nb = sd.nb, nq = sd.nq;
+    if (nb > evr::kMaxNb) {  // only streamed terms hold such a slot
+      oB[s] = oW[s] = oI[s] = oO[s] = oF[s] = 0;
+      continue;
+    }
+    const double *B = h.bw.data() + sd.offB, *W = h.bw.data() + sd.offW, *K = h.keo.data() + sd.offK;
+    std::vector<long double> U((size_t)nb * nb, 0.0L), lam(nb, 0.0L);
+    for (int i = 0; i < nb; ++i) U[i + (size_t)nb * i] = 1.0L;
+    if (hasA) {
+      const double *Q = K + (size_t)evr::kQ * nb * nb;
+      std::vector<long double> q((size_t)nb * nb);
+      double qmax = 0.0;
+      for (int i = 0; i < nb * nb; ++i) qmax = std::max(qmax, std::fabs(Q[i]));
+      for (int i = 0; i < nb; ++i)
+        for (int j = 0; j < nb; ++j) {
+          if (std::fabs(Q[i + nb * j] - Q[j + nb * i]) > 1e-13 * qmax) return EVR_OK;
+          q[i + (size_t)nb * j] = 0.5L * ((long double)Q[i + nb * j] + Q[j + nb * i]);
+        }
+      jacobi_eig(nb, q, U, lam);
+    }
+    auto put = [&](int rows, int cols, auto val) {
+      const int o = (int)pool.size();
+      for (int r = 0; r < rows; ++r)
+        for (int c = 0; c < cols; ++c) pool.push_back((double)val(r, c));
+      while (pool.size() & 1) pool.push_back(0.0);  // 16-byte aligned matrices
+      return o;
+    };
+    oB[s] = put(nq, nb, [&](int r, int c) {
+      long double v = 0.0L;
+      for (int k = 0; k < nb; ++k) v += (long double)B[r + (size_t)nq * k] * U[k + (size_t)nb * c];
+      return v;
+    });
+    oW[s] = put(nb, nq, [&](int r, int c) {
+      long double v = 0.0L;
+      for (int k = 0; k < nb; ++k) v += U[k + (size_t)nb * r] * W[k + (size_t)nb * c];
+      return v;
+    });
+    oI[s] = put(nb, nb, [&](int r, int c) { return U[c + (size_t)nb * r]; });
+    oO[s] = put(nb, nb, [&](int r, int c) { return U[r + (size_t)nb * c]; });
+    // U^T F U
+    auto rot = [&](std::vector<long double> F) {
+      std::vector<long double> t((size_t)nb * nb, 0.0L), o((size_t)nb * nb, 0.0L);
+      for (int i = 0; i < nb; ++i)
+        for (int j = 0; j < nb; ++j)
+          for (int k = 0; k < nb; ++k) t[i + (size_t)nb * j] += F[i + (size_t)nb * k] * U[k + (size_t)nb * j];
+      for (int i = 0; i < nb; ++i)
+        for (int j = 0; j < nb; ++j)
+          for (int k = 0; k < nb; ++k) o[i + (size_t)nb * j] += U[k + (size_t)nb * i] * t[k + (size_t)nb * j];
+      return o;
+    };
+    auto factor = [&](int f) {
+      return std::vector<long double>(K + (size_t)f * nb * nb, K + (size_t)(f + 1) * nb * nb);
+    };
+    std::vector<long double> P = rot(factor(evr::kP)), T = rot(factor(kTd)), Uf, RS;
+    if (hasA) {
+      const int d = s / h.nlev;  // the slot's mode (no compaction with Ga)
+      std::vector<long double> u = factor(evr::kU), r = factor(evr::kR), q = factor(evr::kS);
+      for (size_t i = 0; i < u.size(); ++i) {
+        u[i] *= A(d, d, d);
+        r[i] += q[i];
+      }
+      Uf = rot(u);
+      RS = rot(r);
+    } else {
+      Uf.assign((size_t)nb * nb, 0.0L);
+      RS.assign((size_t)nb * nb, 0.0L);
+    }
+    oF[s] = (int)fac.size();
+    for (int r = 0; r < nb; ++r)
+      for (int c = 0; c < nb; ++c)
+        for (const auto *M : {&P, &T, &Uf, &RS}) fac.push_back((double)(*M)[r + (size_t)nb * c]);
+    for (int c = 0; c < nb; ++c) fac.push_back((double)lam[c]);
+    if (fac.size() & 1) fac.push_back(0.0);  // 16-byte aligned factor rows
+  }
+  // ---- coefficients by position of a set
+  auto c2 = [&](int cix, int a, int b) -> double {
+    const std::vector<int> &m = h.sets[cix];
+    if (m[a] >= 0 && m[b] >= 0) return h.cC[(size_t)m[a] * Dm + m[b]];
+    return (a == b && m[a] == -1) ? 1.0 : 0.0;
+  };
+  auto f1 = [&](int cix, int a) { return (!h.cF1.empty() && h.sets[cix][a] >= 0) ? h.cF1[h.sets[cix][a]] : 0.0; };
+  p->ht_hasM = hasA || !h.cF1.empty();
+  for (int i = 0; i < Dm && !p->ht_hasM; ++i)
+    for (int j = 0; j < Dm; ++j)
+      if (i != j && h.cC[(size_t)i * Dm + j] != 0.0) p->ht_hasM = true;
+
+  // ---- terms
+  std::vector<evr::HTerm> ht(p->nterms);
+  std::vector<evr::HGroup> groups;
+  std::vector<double> coef;
+  std::map<std::vector<int>, int> coef_of;
+  std::vector<int> cap(p->nterms, -1);
+  std::vector<double> cost(p->nterms, 0.0);
+  std::vector<size_t> words_fix(p->nterms, 0), words_vec(p->nterms, 0);
+  std::vector<int> rest[kNumClasses];
+  constexpr size_t kLimit = 160 * 1024 / 8;
+  for (int64_t t = 0; t < p->nterms; ++t) {
+    const evr::TermDev &td = p->terms[t];
+    const int c = p->tclass[t];
+    if (c < 0) continue;  // streamed
+    evr::HTerm &H = ht[t];
+    H.off_nb = td.off_nb;
+    H.off_vq = td.off_vq;
+    H.w = td.w;
+    H.nbt = td.nbt;
+    int nb[evr::kMaxDev], nq[evr::kMaxDev], st[evr::kMaxDev];
+    for (int d = 0, s = 1; d < D; ++d) {
+      nb[d] = p->slots[td.slot[d]].nb;
+      nq[d] = p->slots[td.slot[d]].nq;
+      st[d] = s;
+      s *= nb[d];
+    }
+    // groups over the modes with more than one function
+    H.g0 = (int)groups.size();
+    std::vector<int> gm0, gm1;  // modes of every group (gm1: -1 for a single mode)
+    for (int j = 0; j < td.Dv;) {
+      const int d = td.vmode[j];
+      const int e = j + 1 < td.Dv ? td.vmode[j + 1] : -1;
+      evr::HGroup G{};
+      if (e >= 0 && hgroup_kind(nb[d], nq[d], nb[e], nq[e]) != evr::kHgGeneric) {
+        G.kind = hgroup_kind(nb[d], nq[d], nb[e], nq[e]);
+        gm1.push_back(e);
+      } else {
+        G.kind = hgroup_kind(nb[d], nq[d], 1, 1);
+        gm1.push_back(-1);
+      }
+      gm0.push_back(d);
+      G.nb = nb[d];
+      G.nq = nq[d];
+      G.n1 = st[d];
+      for (int k = 0; k < (gm1.back() >= 0 ? 2 : 1); ++k) {
+        const int s = td.slot[k ? e : d];
+        if (k) {
+          G.nb *= nb[e];
+          G.nq *= nq[e];
+        }
+        G.mB[k] = oB[s];
+        G.mW[k] = oW[s];
+        G.mI[k] = oI[s];
+        G.mO[k] = oO[s];
+        G.pw[k] = oO[s] + p->slots[s].nb * p->slots[s].nb - oB[s];
+      }
+      j += gm1.back() >= 0 ? 2 : 1;
+      groups.push_back(G);
+    }
+    H.ng = (int)groups.size() - H.g0;
+    // pencil mode: the slowest active mode of three functions
+    std::vector<int> act(td.amode, td.amode + td.na);
+    H.na = td.na;
+    H.nbp = 1;
+    for (int k = H.na - 1; k >= 0 && H.nbp == 1; --k)
+      if (nb[act[k]] == 3) {
+        H.nbp = 3;
+        std::rotate(act.begin(), act.begin() + k, act.begin() + k + 1);
+      }
+    if (p->hasKeo && H.na > evr::kHtModes) {
+      rest[c].push_back((int)t);
+      continue;
+    }
+    if (!p->hasKeo) {
+      H.na = 0;
+      H.nbp = 1;
+    }
+    int fw = 0;
+    for (int k = 0; k < H.na; ++k) {
+      const int d = act[k];
+      H.nb[k] = nb[d];
+      H.st[k] = st[d];
+      H.rst[k] = 1.0f / (float)st[d];
+      H.rnb[k] = 1.0f / (float)nb[d];
+      H.gF[k] = oF[td.slot[d]];
+      H.lF[k] = fw;
+      fw += 4 * nb[d] * nb[d] + nb[d];
+      fw += fw & 1;
+    }
+    H.lC = fw;
+    if (p->hasKeo) fw += evr::hcoef_words(H.na);
+    H.fw = fw;
+    // coefficient rows of this active list (and its one-function slots)
+    {
+      std::vector<int> key{td.cix, H.na, H.nbp};
+      for (int k = 0; k < H.na; ++k) key.push_back(act[k]);
+      std::vector<char> is_act(D, 0);
+      for (int k = 0; k < H.na; ++k) is_act[act[k]] = 1;
+      for (int d = 0; d < D; ++d)
+        if (!is_act[d]) key.push_back(td.slot[d]);
+      auto it = coef_of.find(key);
+      if (it == coef_of.end()) {
+        const int na = H.na, RL = evr::hrow_len(na);
+        const bool pen = H.nbp > 1;
+        const size_t o = coef.size();
+        coef.resize(o + evr::hcoef_words(na), 0.0);
+        double *rows = coef.data() + o;
+        auto set = [&](int row, int k, double v) { rows[(size_t)row * RL + (pen && k == 0 ? na + 1 : k)] += v; };
+        // one-function modes with vanishing P, Q, R: scalars (their U and
+        // R + S factors with the coefficients of a q-linear G)
+        for (int i = 0; i < D && p->hasKeo; ++i) {
+          if (is_act[i]) continue;
+          const double *K = h.keo.data() + p->slots[td.slot[i]].offK;
+          rows[na] += c2(td.cix, i, i) * K[kTd];
+          if (hasA) {
+            rows[na] += A(i, i, i) * K[evr::kU];
+            for (int k = 0; k < na; ++k) set(0, k, A(i, i, act[k]) * K[kTd]);
+          }
+        }
+        double *alpha = rows + (size_t)(1 + na + na * (na - 1) / 2) * RL, *fs = alpha + na * na;
+        for (int j = 0; j < na; ++j) {
+          const int mj = act[j];
+          rows[(size_t)(1 + j) * RL + na] = c2(td.cix, mj, mj);
+          if (hasA)
+            for (int k = 0; k < na; ++k)
+              if (k != j) set(1 + j, k, A(mj, mj, act[k]));
+          for (int i = 0; i < na; ++i) {
+            if (i == j) continue;
+            const int mi = act[i];
+            if (i < j) {
+              const int row = 1 + na + j * (j - 1) / 2 + i;
+              rows[(size_t)row * RL + na] = c2(td.cix, mi, mj) + c2(td.cix, mj, mi);
+              if (hasA)
+                for (int k = 0; k < na; ++k)
+                  if (k != i && k != j) set(row, k, A(mi, mj, act[k]) + A(mj, mi, act[k]));
+            }
+            if (hasA) alpha[j * na + i] = A(mi, mj, mj);
+          }
+          fs[j] = f1(td.cix, mj);
+          if (hasA)
+            for (int i = 0; i < D; ++i)
+              if (!is_act[i])
+                fs[j] += A(mj, i, i) * h.keo[p->slots[td.slot[i]].offK + evr::kS];
+        }
+        it = coef_of.emplace(key, (int)o).first;
+      }
+      H.coef = it->second;
+    }
+    // LDS: x, y and the larger of the V buffers and the M arrays
+    const size_t nbt = td.nbt;
+    auto vwords = [&](int nO, int &wA, int &wB, int &nbI, int &nbO) -> size_t {
+      const int gi = H.ng - nO;
+      nbI = 1;
+      nbO = 1;
+      for (int g = 0; g < H.ng; ++g) (g < gi ? nbI : nbO) *= groups[H.g0 + g].nb;
+      wA = wB = 0;
+      int64_t cur = nbI;
+      for (int g = 0; g + 1 < gi; ++g) {
+        cur = cur / groups[H.g0 + g].nb * groups[H.g0 + g].nq;
+        int &w = (g & 1) ? wB : wA;
+        w = (int)std::max<int64_t>(w, cur);
+      }
+      return (size_t)wA + wB + (nO ? (size_t)nbI : 0);
+    };
+    const int nM = p->hasKeo && p->ht_hasM ? std::max(0, H.na - (H.nbp > 1 ? 1 : 0)) : 0;
+    bool fits = false;
+    size_t wv = 0, wfix = fw;
+    for (int nO = 0; nO <= std::max(0, H.ng - 1) && !fits; ++nO) {
+      int wA, wB, nbI, nbO, nOm = 0;
+      const size_t vw = vwords(nO, wA, wB, nbI, nbO);
+      const size_t cr = nO ? 2 * (size_t)nbO : 0;
+      if (fw + 2 * nbt + vw + cr > kLimit) continue;
+      H.nO = nO;
+      H.nbO = nbO;
+      H.nbI = nbI;
+      H.wA = wA;
+      H.wB = wB;
+      H.QO = 1;
+      for (int g = H.ng - nO; g < H.ng; ++g) {
+        const evr::HGroup &G = groups[H.g0 + g];
+        H.QO *= G.nq;
+        for (int k = 0; k < 2; ++k) {
+          const int d = k ? gm1[g] : gm0[g];
+          if (d < 0) continue;
+          if (nOm < 4) {
+            H.oB[nOm] = G.mB[k];
+            H.oW[nOm] = G.mW[k];
+            H.onb[nOm] = nb[d];
+            H.onq[nOm] = nq[d];
+          }
+          ++nOm;
+        }
+      }
+      H.nOm = nOm;
+      if (nOm > 4) break;
+      wv = 2 * nbt + vw;
+      wfix = fw + cr;
+      H.nm = nM;
+      while (H.nm > 1 && fw + (2 + (size_t)H.nm) * nbt > kLimit) --H.nm;
+      if (nM && fw + 3 * nbt > kLimit) break;
+      wv = std::max(wv, (2 + (size_t)H.nm) * nbt);
+      fits = wfix + wv <= kLimit;
+    }
+    if (!fits) {
+      rest[c].push_back((int)t);
+      continue;
+    }
+    for (int k = 0; k < kHtCaps; ++k)
+      if (8 * (wfix + (wv << kHtClasses[k].lv)) <= (size_t)kHtClasses[k].lds) cap[t] = k;
+    words_fix[t] = wfix;
+    words_vec[t] = wv;
+    cost[t] = (double)nbt * (4.0 + H.na * H.na + 2.0 * H.ng) * H.QO;
+  }
+  // ---- work list by class, most expensive terms first
+  std::vector<int> order;
+  for (int k = 0; k < kHtCaps; ++k) {
+    std::vector<int> ids;
+    for (int64_t t = 0; t < p->nterms; ++t)
+      if (cap[t] == k) ids.push_back((int)t);
+    std::stable_sort(ids.begin(), ids.end(), [&](int a, int b) { return cost[a] > cost[b]; });
+    p->ht_items[k] = 0;
+    for (int l = 0; l < 4; ++l) p->ht_lds[k][l] = 0;
+    for (int t : ids) {
+      for (int l = 0; l <= kHtClasses[k].lv; ++l)
+        p->ht_lds[k][l] = std::max(p->ht_lds[k][l], 8 * (words_fix[t] + (words_vec[t] << l)));
+      p->ht_items[k] = std::max(p->ht_items[k], ht[t].nbt / ht[t].nbp);
+    }
+    while (ids.size() % 8) ids.push_back(-1);
+    p->ht_off[k] = (int64_t)order.size();
+    order.insert(order.end(), ids.begin(), ids.end());
+  }
+  p->ht_off[kHtCaps] = (int64_t)order.size();
+  for (int c = 0; c < kNumClasses; ++c) {
+    while (rest[c].size() % 8) rest[c].push_back(-1);
+    p->ht_nrest[c] = (int64_t)rest[c].size();
+    HIP_TRY(p->d_ht_rest[c].upload(rest[c].data(), rest[c].size(), p->stream));
+  }
+  HIP_TRY(p->d_ht.upload(ht.data(), ht.size(), p->stream));
+  HIP_TRY(p->d_hg.upload(groups.data(), groups.size(), p->stream));
+  HIP_TRY(p->d_hpool.upload(pool.data(), pool.size(), p->stream));
+  HIP_TRY(p->d_hfac.upload(fac.data(), fac.size(), p->stream));
+  HIP_TRY(p->d_hcoef.upload(coef.data(), coef.size(), p->stream));
+  HIP_TRY(p->d_horder.upload(order.data(), order.size(), p->stream));
+  p->ht_on.resize(p->nterms);
+  for (int64_t t = 0; t < p->nterms; ++t) p->ht_on[t] = cap[t] >= 0;
+  p->ht = true;
+  return EVR_OK;
+}
+
+// The register-block terms of an FP64 H|psi>: one launch per class.  A block
+// of few vectors takes fewer per workgroup (nvec rounded up to a power of
+// two); classes that then agree in it share a launch when their workgroups
+// are too few to fill the device one class at a time.
+int run_hterms(evr_plan *p, int nvec, const double *X, double *R)
+{
+  int want = 0;
+  while (want < 3 && (1 << want) < nvec) ++want;
+  evr::HArgs a{};
+  a.nvec = nvec;
+  a.hasV = p->hasV;
+  a.hasKeo = p->hasKeo;
+  a.hasA = p->hasA;
+  a.hasM = p->ht_hasM;
+  a.terms = (const evr::HTerm EVR_CONST *)p->d_ht.ptr;
+  a.groups = (const evr::HGroup EVR_CONST *)p->d_hg.ptr;
+  a.pool = (evr::ctab)p->d_hpool.ptr;
+  a.fpool = p->d_hfac.ptr;
+  a.coef = p->d_hcoef.ptr;
+  a.map = p->d_map.ptr;
+  a.rowpos = p->d_rowpos.ptr;
+  a.V = p->d_Veff.ptr;
+  a.X = X;
+  a.R = R;
+  for (int lo = 0; lo < kHtCaps;) {
+    a.lv = std::min(kHtClasses[lo].lv, want);
+    const int64_t tiles = (nvec + (1 << a.lv) - 1) >> a.lv;
+    size_t lds = p->ht_lds[lo][a.lv];
+    int items = p->ht_items[lo] << a.lv, hi = lo + 1, nt = kHtClasses[lo].nt;
+    while (hi < kHtCaps && std::min(kHtClasses[hi].lv, want) == a.lv &&
+           (p->ht_off[hi + 1] - p->ht_off[lo]) * tiles <= 4 * p->ncu) {
+      lds = std::max(lds, p->ht_lds[hi][a.lv]);
+      items = std::max(items, p->ht_items[hi] << a.lv);
+      ++hi;
+    }
+    const int64_t units = p->ht_off[hi] - p->ht_off[lo];
+    if (units > 0) {
+      while (nt > 64 && nt / 2 >= items) nt /= 2;
+      const int64_t nblk = units * tiles;
+      a.order = (const int EVR_CONST *)(p->d_horder.ptr + p->ht_off[lo]);
+      const hipError_t e = evr::launch_hterm(a, nblk, nt, lds, p->stream);
+      if (e != hipSuccess) return fail(EVR_ERR_HIP, std::string("term kernel: ") + hipGetErrorString(e));
+    }
+    lo = hi;
+  }
+  return EVR_OK;
+}
+
+// Ends the bracket opened on the slot's first event and books its time.
+void profile_slot(evr_plan *p, int slot, double flops)
+{
+  (void)hipEventRecord(p->ev[2 * slot + 1], p->stream);
+  (void)hipEventSynchronize(p->ev[2 * slot + 1]);
+  float ms = 0.f;
+  (void)hipEventElapsedTime(&ms, p->ev[2 * slot], p->ev[2 * slot + 1]);
+  p->ms_acc[slot] += ms;
+  p->flops_acc[slot] += flops;
+  p->launches[slot] += 1;
+}
+
 // Apply every term class for `nvec` vectors held in X ([nb_packed][nvec]).
 template <typename T>
 int run_terms(evr_plan *p, int mode, int nvec, const T *X, T *R, T *G, const T *Gin, const T *bw,
@@ -603,12 +1115,23 @@ int run_terms(evr_plan *p, int mode, int nvec, const T *X, T *R, T *G, const T *
 {
   if (!p->one.empty() && !diagKeo && (mode == evr::kModeHpsi || mode == evr::kModeB2G || mode == evr::kModeG2B))
     return run_streamed<T>(p, p->one, mode, nvec, X, R, G, Gin);
+  bool blocks = false;  // the terms in register blocks; the classes keep the rest
+  if constexpr (sizeof(T) == 8) {
+    blocks = p->ht && mode == evr::kModeHpsi;
+    if (blocks) {
+      if (p->profiling) (void)hipEventRecord(p->ev[2 * kProfHt], p->stream);
+      const int rc = run_hterms(p, nvec, X, R);
+      if (rc) return rc;
+      if (p->profiling) profile_slot(p, kProfHt, p->flops_ht * nvec);
+    }
+  }
   for (int c = 0; c < kNumClasses; ++c) {
-    if (p->nunits[c] == 0) continue;
+    const int64_t units = blocks ? p->ht_nrest[c] : p->nunits[c];
+    if (units == 0) continue;
     evr::TermParams<T> prm = base_params<T>(p, mode, nvec);
     prm.diagKeo = diagKeo;
-    prm.nunits = p->nunits[c];
-    prm.order = p->d_order[c].ptr;
+    prm.nunits = units;
+    prm.order = blocks ? p->d_ht_rest[c].ptr : p->d_order[c].ptr;
     prm.bw = bw;
     prm.keo = keo;
     prm.V = V;
@@ -618,17 +1141,9 @@ int run_terms(evr_plan *p, int mode, int nvec, const T *X, T *R, T *G, const T *
     prm.Gin = Gin;
     size_t lds = sizeof(T) == 8 ? p->lds_bytes64[c] : p->lds_bytes32[c];
     if (p->profiling) (void)hipEventRecord(p->ev[2 * c], p->stream);
-    hipError_t e = launch_class<T>(c, prm, p->nunits[c], nvec, lds, p->stream);
+    hipError_t e = launch_class<T>(c, prm, units, nvec, lds, p->stream);
     if (e != hipSuccess) return fail(EVR_ERR_HIP, std::string("term kernel: ") + hipGetErrorString(e));
-    if (p->profiling) {
-      (void)hipEventRecord(p->ev[2 * c + 1], p->stream);
-      (void)hipEventSynchronize(p->ev[2 * c + 1]);
-      float ms = 0.f;
-      (void)hipEventElapsedTime(&ms, p->ev[2 * c], p->ev[2 * c + 1]);
-      p->ms_acc[c] += ms;
-      p->flops_acc[c] += p->flops_class[c] * nvec;
-      p->launches[c] += 1;
-    }
+    if (p->profiling) profile_slot(p, c, (blocks ? p->flops_rest[c] : p->flops_class[c]) * nvec);
   }
   if (!p->big.empty()) {
     if (diagKeo) return fail(EVR_ERR_ARG, "the kinetic diagonal of a streamed term is not formed here");
@@ -776,19 +1291,10 @@ std::vector<int2> asm_items(const std::vector<int> &nbt)
 template <typename T>
 hipError_t apply_assembled(evr_plan *p, const T *A, const T *X, int nvec, T *R)
 {
-  const int slot = kNumClasses;  // profiling slot of the assembled apply
-  if (p->profiling) (void)hipEventRecord(p->ev[2 * slot], p->stream);
+  if (p->profiling) (void)hipEventRecord(p->ev[2 * kProfAsm], p->stream);
   const hipError_t e = apply_op<T>(plan_op(p), A, X, nvec, R);
   if (e != hipSuccess) return e;
-  if (p->profiling) {
-    (void)hipEventRecord(p->ev[2 * slot + 1], p->stream);
-    (void)hipEventSynchronize(p->ev[2 * slot + 1]);
-    float ms = 0.f;
-    (void)hipEventElapsedTime(&ms, p->ev[2 * slot], p->ev[2 * slot + 1]);
-    p->ms_acc[slot] += ms;
-    p->flops_acc[slot] += p->asm_flops_per_vec * nvec;
-    p->launches[slot] += 1;
-  }
+  if (p->profiling) profile_slot(p, kProfAsm, p->asm_flops_per_vec * nvec);
   return hipSuccess;
 }
 
@@ -1444,6 +1950,8 @@ int evr_plan_create(const evr_basis_desc *bd, const evr_op_desc *op, int max_nve
   {
     const int rc = apply_classes(p.get());
     if (rc) return rc;
+    const int rch = build_hterms(p.get(), HtInput{bw, keo, cC, cA, cF1, sets, D, nlev});
+    if (rch) return rch;
   }
 
   // ---- deterministic scatter: the term rows of packed function pk, in
@@ -1846,9 +2354,15 @@ int evr_plan_release_assembled(evr_plan *p)
 
 static void recount_flops(evr_plan *p)
 {
-  for (int c = 0; c < kNumClasses; ++c) p->flops_class[c] = 0;
-  for (int64_t t = 0; t < p->nterms; ++t)
-    if (p->tclass[t] >= 0) p->flops_class[p->tclass[t]] += term_flops(p, p->terms[t]);
+  for (int c = 0; c < kNumClasses; ++c) p->flops_class[c] = p->flops_rest[c] = 0;
+  p->flops_ht = 0;
+  for (int64_t t = 0; t < p->nterms; ++t) {
+    if (p->tclass[t] < 0) continue;
+    const double f = term_flops(p, p->terms[t]);
+    p->flops_class[p->tclass[t]] += f;
+    if (p->ht && p->ht_on[t]) p->flops_ht += f;
+    else p->flops_rest[p->tclass[t]] += f;
+  }
 }
 
 int evr_plan_autotune(evr_plan *p, int nvec, int flags, int reps, int *chosen, double *ms_static,
@@ -1963,7 +2477,8 @@ int evr_plan_set_profiling(evr_plan *p, int on)
   if (on && !p->ev[0])
     for (auto &e : p->ev) HIP_TRY(hipEventCreate(&e));
   p->profiling = on != 0;
-  for (int c = 0; c <= kNumClasses; ++c) p->ms_acc[c] = p->flops_acc[c] = 0, p->launches[c] = 0;
+  for (int c = 0; c < kProfSlots; ++c) p->ms_acc[c] = p->flops_acc[c] = 0, p->launches[c] = 0;
+  recount_flops(p);
   return EVR_OK;
 }
 
@@ -1982,11 +2497,12 @@ int evr_plan_kernel_stats(evr_plan *p, int max, char *names, double *ms, double 
     if (launches) launches[k] = p->launches[c];
     ++k;
   }
-  if (p->launches[kNumClasses] > 0 && k < max) {
-    if (names) snprintf(names + 64 * k, 64, "k_apply_asm");
-    if (ms) ms[k] = p->ms_acc[kNumClasses];
-    if (flops) flops[k] = p->flops_acc[kNumClasses];
-    if (launches) launches[k] = p->launches[kNumClasses];
+  for (int c : {kProfAsm, kProfHt}) {
+    if (p->launches[c] == 0 || k >= max) continue;
+    if (names) snprintf(names + 64 * k, 64, c == kProfAsm ? "k_apply_asm" : "k_hterm");
+    if (ms) ms[k] = p->ms_acc[c];
+    if (flops) flops[k] = p->flops_acc[c];
+    if (launches) launches[k] = p->launches[c];
     ++k;
   }
   *n = k;
@@ -2010,7 +2526,8 @@ static int ensure_v32(evr_plan *p)
 // takes its number of waves of workgroups (units x ceil(nvec / nvw) over the
 // 1024 / nt workgroups each CU holds, fewer when LDS is short) times one
 // workgroup's time, and a workgroup always does nvw vectors' work, padded or
-// not.  The per-workgroup rates below are the classes' whole-device TFLOP/s
+// not (FP32, and FP64 plans that keep the term kernels).  The per-workgroup
+// rates below are the classes' whole-device TFLOP/s
 // measured at D=9 SG4 L=8 with 32 vectors, wave-count corrected; the model
 // then gives 8.7 / 10.4 / 17.0 / 31.2 / 119.7 ms for 1 / 2 / 4 / 8 / 32
 // vectors there (measured 9.1 / 10.8 / 17.2 / 31.6 / 120.5) and overestimates
@@ -2018,8 +2535,24 @@ static int ensure_v32(evr_plan *p)
 // model is taken: at D=9 L=8 FP64 the sum-factorised one up to 5 vectors (17.3
 // against 22.5 ms at 4, 23.3 against 22.8 at 5), at D=12 L=6 the assembled
 // one from 1 vector (2.49 against 2.79 ms).
+//
+// FP64 plans whose terms all run in register blocks (k_hterm) cost, measured
+// at D=9 SG4 L=8 and D=12 SG4 L=6 with 1 to 32 vectors, about 68 ps per term
+// function and vector plus 50 ps per term function and 45 us per call (1.77 /
+// 4.8 / 16.7 / 32.6 ms by the model for 1 / 4 / 16 / 32 vectors at D=9 L=8,
+// measured 1.76 / 4.42 / 16.2 / 32.4); the assembled call adds its term rows
+// to the pool (23.2 ms for one vector, 26.4 ms for 32).  There the
+// sum-factorised path is taken up to 25 vectors (24.6 against 27.6 ms) and up
+// to 7 at D=12 L=6 (1.93 against 2.75 ms); at D=6 SG4 L=5, where both are
+// latency, the assembled one from 1 vector (0.030 against 0.057 ms).
 static bool matrix_free_cheaper(const evr_plan *p, int nvec, bool fp32)
 {
+  bool ht = p->ht && !fp32;
+  for (int c = 0; c < kNumClasses; ++c) ht = ht && p->ht_nrest[c] == 0;
+  if (ht) {
+    const double n = (double)p->sum_nb;
+    return 4.5e-5 + n * (6.8e-11 * nvec + 5.0e-11) < p->asm_bytes64 / 6.0e12 + n * nvec * 4.8e-12 + 2.4e-5;
+  }
   constexpr double kClassTflops[] = {1.23, 1.82, 2.56, 2.88, 3.83, 5.17, 4.70, 1.99};
   static_assert(sizeof(kClassTflops) / sizeof(double) == kNumClasses, "one rate per term class");
   double t_mf = 8e-6 * 2;  // gather-free pack + reduction

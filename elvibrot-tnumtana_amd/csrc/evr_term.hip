@@ -76,17 +76,6 @@ __device__ __forceinline__ StepDev uniform_step(const StepDev &s)
   return r;
 }
 
-// Integer division of x < 2^24 by a wave-uniform d via the float reciprocal
-// (exact after one correction step).
-__device__ __forceinline__ int fdiv(int x, int d, float rd)
-{
-  int q = (int)((float)x * rd);
-  int r = x - q * d;
-  if (r < 0) --q;
-  else if (r >= d) ++q;
-  return q;
-}
-
 // out[(i1 + n1*(q + nout*i3))*NVW + v] = sum_k M[q + nout*k] in[(i1 + n1*(k + nin*i3))*NVW + v]
 // M is read from global memory at wave-uniform addresses (scalar loads, the
 // coefficients live in SGPRs); sizes known at compile time are fully unrolled

@@ -306,7 +306,9 @@ int evr_coupled_oppsi(evr_coupled *c, int nvec, const double *psi, double *hpsi,
  * at the first slower one.  The layout chosen stays with the plan
  * (evr_oppsi, the assembly).  chosen (EVR_NCLASSES ints, or NULL): the class
  * of each bucket; ms_static / ms_tuned: the H|psi> times of the static rule
- * and of the tuned layout.  Results are unchanged by the layout (the same
+ * and of the tuned layout.  The classes carry FP32 H|psi>, the assembly and
+ * the transforms; FP64 H|psi> runs in register blocks of its own except on
+ * terms that those do not take, so its two times agree.  Results are unchanged by the layout (the same
  * arithmetic per term). */
 #define EVR_NCLASSES 8
 int evr_plan_autotune(evr_plan *p, int nvec, int flags, int reps, int *chosen, double *ms_static,

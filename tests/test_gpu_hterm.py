@@ -1,0 +1,51 @@
+"""H|psi> of the Smolyak terms in register blocks against the oracle: every
+group shape of the kernel and the generic one (the 1D laws 1 + 2l functions on
+2 + 2l or 1 + 2l points, 1 + l on 2 + l, 2 + 2l on 3 + 2l; slots up to 19
+functions), terms of one function, terms whose V part runs in slabs (seven
+active modes), one to nine vectors, the kinetic part with and without a
+q-linear G and off-diagonal terms, and a G(q) that is not symmetric in its two
+indices, which the older term kernels keep."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+TOL64 = 1e-12  # the parity bar of every FP64 H|psi> test
+
+CASES = [(1, 3, (1, 2, 2, 2), 10, "ga", 1), (2, 9, (1, 2, 2, 2), 10, "ga", 1), (3, 6, (1, 2, 2, 2), 10, "ga", 4),
+         (4, 4, (1, 2, 2, 2), 10, "ga", 3), (4, 4, (1, 2, 1, 2), 10, "ga", 1), (4, 3, (1, 1, 2, 1), 10, "ga", 2),
+         (3, 3, (2, 2, 3, 2), 10, "ga", 9), (6, 5, (1, 2, 2, 2), 10, "ga", 2), (6, 4, (1, 2, 2, 2), 10, "ga", 7),
+         (4, 4, (1, 2, 2, 2), 10, "g0", 3), (4, 4, (1, 2, 2, 2), 10, "off", 3), (4, 3, (1, 2, 1, 2), 1, "type1", 2),
+         (4, 4, (1, 2, 2, 2), 0, "v", 2), (5, 4, (1, 2, 2, 2), 10, "skew", 2), (7, 7, (1, 2, 2, 2), 10, "ga", 1)]
+
+
+@pytest.mark.parametrize("D,L,law,type_,kind,nvec", CASES)
+def test_hterm(evr, oracle_mod, D, L, law, type_, kind, nvec):
+    rng = np.random.RandomState(D * 100 + L)
+    s = oracle_mod.SG4(D, L, L, *law)
+    b = evr.Basis.sg4(D, L, L, *law)
+    G0 = np.diag(rng.uniform(1.0, 3.0, D))
+    if kind != "g0":
+        G0 = G0 + 0.1 * rng.uniform(-1.0, 1.0, (D, D))
+    Ga = F1 = None
+    if kind in ("ga", "skew"):
+        Ga = rng.uniform(-0.1, 0.1, (D, D, D))
+        if kind == "ga":
+            Ga = 0.5 * (Ga + Ga.transpose(1, 0, 2))  # G_ij(q) = G_ji(q)
+        Ga = Ga.ravel(order="F")
+    if type_ == 1:
+        F1 = rng.uniform(-0.1, 0.1, D)
+    q = s.grid()
+    V = 0.5 * (q ** 2).sum(axis=1) + 0.1 * q[:, 0] * q[:, -1] ** 2
+    X = np.asfortranarray(rng.randn(b.nb_packed, nvec))
+    if type_ == 10:
+        op, kw = oracle_mod.Op(10, V=V, G0=G0, Ga=Ga), dict(G0=G0, Ga=Ga)
+    elif type_ == 1:
+        op, kw = oracle_mod.Op(1, V=V, F2=G0, F1=F1), dict(F2=G0, F1=F1)
+    else:
+        op, kw = oracle_mod.Op(0, V=V), {}
+    ref = s.oppsi(op, X)
+    plan = evr.Plan(b, type=type_, V=V, max_nvec=nvec, **kw)
+    e = np.abs(plan.TabOpPsi(X) - ref).max() / np.abs(ref).max()
+    print("D=%d L=%d law %s type %d %s, %d vectors: %.2e" % (D, L, law, type_, kind, nvec, e))
+    assert e < TOL64
