@@ -462,7 +462,7 @@ def transforms_run(args):
     g = plan.BasisRep_TO_GridRep(x)          # warm-up (allocates the grid buffer)
     plan.GridRep_TO_BasisRep(g)
     plan.set_profiling(True)
-    ms = lambda: sum(s[1] for s in plan.kernel_stats() if s[0].startswith("k_term"))
+    ms = lambda: sum(s[1] for s in plan.kernel_stats() if s[0].startswith(("k_term", "k_b2g", "k_g2b")))
     m0 = ms()
     g = plan.BasisRep_TO_GridRep(x)
     m1 = ms()

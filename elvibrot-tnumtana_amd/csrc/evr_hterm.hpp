@@ -37,6 +37,7 @@ struct HGroup {
   int mB[2], mW[2];     // 1D matrices in the pool (row-major): B (nq x nb), W (nb x nq)
   int mI[2], mO[2];     // rotation in (U^T) and out (U), nb x nb
   int pw[2];            // words of the mode's four matrices (B first, contiguous)
+  int mP[2], mQ[2];     // B and W without the rotation (the transforms)
 };
 
 // One term.  Active positions (modes whose P, Q, R do not vanish) in the
@@ -66,6 +67,38 @@ struct HTerm {  // sizeof: a multiple of 8
 #endif
 using ctab = const double EVR_CONST *;
 
+// One term of the basis <-> grid transforms.  The full grid point p = pl + Pl
+// ph splits into the first nlow modes (pl) and the others (ph); each side into
+// the points r of its modes with more than one function and the points c of
+// its one-function modes, pl = Rl-part + Cl-part.
+struct XTerm {  // sizeof: a multiple of 8
+  int64_t off_nb, off_nq;  // term rows, first point of the term grid
+  double w;                // weight of the G->B scatter (0 below 1e-6, BGSG4:1004)
+  int nbt, nqt, nvq;       // functions, points, points of the modes with more than one function
+  int ng, g0;              // groups and the first of them
+  int nlow, D;             // modes of the low part, modes
+  int Pl, Ph, Rl, Rh;      // points of the low and high parts, of their r parts
+  int wA, wB;              // LDS words of the two tensor buffers, B->G
+  int uA, uB;              // the same, G->B
+  int nq[kMaxDev];
+  int one[kMaxDev];        // one-function modes: offset of B (nq x 1) in the pool, W (1 x nq) follows; -1 else
+};
+
+struct XArgs {
+  int nvec;
+  const int EVR_CONST *order;      // terms of the workgroups
+  const XTerm EVR_CONST *terms;
+  const HGroup EVR_CONST *groups;
+  ctab pool;
+  const double *pool1;     // B and W of the one-function modes
+  const int *map, *rowpos;
+  const double *X;         // B->G: packed block [function][vector]
+  double *G;               // B->G: grid columns
+  const double *Gin;       // G->B: grid columns
+  double *R;               // G->B: term rows [row][vector]
+  int64_t gld;             // column stride of the grid
+};
+
 // One launch.  The pointers are read from the argument block where they are
 // used, so they do not hold scalar registers over the whole kernel.
 struct HArgs {
@@ -82,6 +115,14 @@ struct HArgs {
   const double *V, *X;
   double *R;
 };
+
+// threads and LDS words of a transform workgroup; high r points a wave of the
+// G->B contraction takes at a time
+constexpr int kXThreads = 256;
+constexpr int kXRows = 2;
+size_t xform_words(const XTerm &t, bool b2g);
+// basis -> grid or grid -> basis on n terms x nvec vectors
+hipError_t launch_xform(const XArgs &a, bool b2g, int64_t nterms, size_t lds, hipStream_t s);
 
 // k_hterm on nblk workgroups of nt threads
 hipError_t launch_hterm(const HArgs &a, int64_t nblk, int nt, size_t lds, hipStream_t s);

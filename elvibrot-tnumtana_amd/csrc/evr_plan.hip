@@ -84,8 +84,10 @@ struct KClass {
 constexpr KClass kClasses[] = {{256, 1, 4},  {512, 1, 4},  {512, 2, 4}, {512, 2, 2},
                                {512, 4, 2}, {512, 4, 1}, {1024, 4, 1}, {1024, 8, 1}};
 constexpr int kNumClasses = sizeof(kClasses) / sizeof(kClasses[0]);
-// profiling slots: the term classes, the assembled apply, the register-block terms
-constexpr int kProfAsm = kNumClasses, kProfHt = kNumClasses + 1, kProfSlots = kNumClasses + 2;
+// profiling slots: the term classes, the assembled apply, the register-block
+// terms and transforms
+constexpr int kProfAsm = kNumClasses, kProfHt = kNumClasses + 1, kProfB2g = kNumClasses + 2, kProfG2b = kNumClasses + 3,
+              kProfSlots = kNumClasses + 4;
 // dynamic LDS per workgroup: 160 KiB less a reserve for the kernels' static
 // arrays (about 2 KiB for the term kernels)
 constexpr size_t kLdsLimit = 160 * 1024 - 4096;
@@ -100,6 +102,9 @@ constexpr int kKiB = 1024;
 constexpr HtClass kHtClasses[] = {{0, 160 * kKiB, 1024}, {0, 80 * kKiB, 512}, {0, 53 * kKiB, 320}, {0, 40 * kKiB, 256},
                                   {1, 40 * kKiB, 256},   {2, 40 * kKiB, 256}, {3, 40 * kKiB, 256}};
 constexpr int kHtCaps = sizeof(kHtClasses) / sizeof(kHtClasses[0]);
+// LDS classes of the transform workgroups (256 threads): 1, 2, 4, 8 per CU
+constexpr int kXLds[] = {160 * kKiB, 80 * kKiB, 40 * kKiB, 20 * kKiB};
+constexpr int kXClasses = sizeof(kXLds) / sizeof(kXLds[0]);
 // a one-term plan of at least this many functions runs its term streamed
 constexpr int kStreamOneMin = 256;
 
@@ -191,6 +196,13 @@ struct evr_plan {
   int64_t ht_off[kHtCaps + 1] = {}, ht_nrest[kNumClasses] = {};
   size_t ht_lds[kHtCaps][4] = {};
   int ht_items[kHtCaps] = {};
+  // FP64 basis <-> grid transforms (evr_xform.hip): terms by LDS class, and
+  // those whose reduced grid exceeds a workgroup (x_rest, term kernels)
+  bool xt = false;
+  DevBuf<evr::XTerm> d_xt;
+  DevBuf<int> d_xorder[2], d_x_rest[2][kNumClasses];  // [grid -> basis, basis -> grid]
+  int64_t x_off[2][kXClasses + 1] = {}, x_nrest[2][kNumClasses] = {};
+  size_t x_lds[2][kXClasses] = {};
   // work buffers
   DevBuf<double> d_X, d_R, d_psi, d_hpsi, d_G;
   DevBuf<double> d_gw;  // w_t * quadrature weight of every term-grid point (lazy)
@@ -230,7 +242,12 @@ struct evr_plan {
     d_GG.release(); d_Jg.release(); d_Sg.release(); d_Gg.release(); d_Pg.release(); d_Fg.release();
     d_F2g.release(); d_F1g.release(); d_gitems.release(); d_dp_perm.release(); d_big.release();
     d_ht.release(); d_hg.release(); d_hpool.release(); d_hfac.release(); d_hcoef.release(); d_horder.release();
-    for (int c = 0; c < kNumClasses; ++c) d_ht_rest[c].release();
+    for (int c = 0; c < kNumClasses; ++c) {
+      d_ht_rest[c].release();
+      d_x_rest[0][c].release();
+      d_x_rest[1][c].release();
+    }
+    d_xt.release(); d_xorder[0].release(); d_xorder[1].release();
     d_Wq.release(); d_As.release(); d_R2.release(); d_F2w.release(); d_F1w.release();
     for (auto &e : ev)
       if (e) (void)hipEventDestroy(e);
@@ -698,39 +715,43 @@ int build_hterms(evr_plan *p, const HtInput &h)
   const int D = p->D, Dm = h.D, ns = (int)p->slots.size();
   const bool hasA = p->hasA;
   auto A = [&](int i, int j, int k) { return h.cA[((size_t)i * Dm + j) * Dm + k]; };
+  bool keo_ok = true;
   if (hasA) {
     double amax = 0.0;
     for (double v : h.cA) amax = std::max(amax, std::fabs(v));
     for (int i = 0; i < Dm; ++i)
-      for (int j = 0; j < Dm; ++j)
-        if (std::fabs(A(j, i, j) - A(i, j, j)) > 4e-16 * amax) return EVR_OK;
+      for (int j = 0; j < Dm; ++j) keo_ok = keo_ok && std::fabs(A(j, i, j) - A(i, j, j)) <= 4e-16 * amax;
+    for (const evr::SlotDev &sd : p->slots) {
+      if (sd.nb > evr::kMaxNb) continue;
+      const double *Q = h.keo.data() + sd.offK + (size_t)evr::kQ * sd.nb * sd.nb;
+      double qmax = 0.0;
+      for (int i = 0; i < sd.nb * sd.nb; ++i) qmax = std::max(qmax, std::fabs(Q[i]));
+      for (int i = 0; i < sd.nb; ++i)
+        for (int j = 0; j < i; ++j)
+          keo_ok = keo_ok && std::fabs(Q[i + sd.nb * j] - Q[j + sd.nb * i]) <= 1e-13 * qmax;
+    }
   }
   // ---- per slot: B, W (rotated with a q-linear G) and the rotations, row by
   // row (a thread's scalar loads take whole rows), and the factor rows
   // [row][col]{P, T, a_jjj U, R + S} followed by xi
   std::vector<double> pool, fac;
-  std::vector<int> oB(ns), oW(ns), oI(ns), oO(ns), oF(ns);
+  std::vector<int> oB(ns), oW(ns), oI(ns), oO(ns), oF(ns), oP(ns), oQ(ns);
   const int kTd = p->diagT2 ? evr::kT2 : evr::kT;
   for (int s = 0; s < ns; ++s) {
     const evr::SlotDev &sd = p->slots[s];
     const int nb = sd.nb, nq = sd.nq;
     if (nb > evr::kMaxNb) {  // only streamed terms hold such a slot
-      oB[s] = oW[s] = oI[s] = oO[s] = oF[s] = 0;
+      oB[s] = oW[s] = oI[s] = oO[s] = oF[s] = oP[s] = oQ[s] = 0;
       continue;
     }
     const double *B = h.bw.data() + sd.offB, *W = h.bw.data() + sd.offW, *K = h.keo.data() + sd.offK;
     std::vector<long double> U((size_t)nb * nb, 0.0L), lam(nb, 0.0L);
     for (int i = 0; i < nb; ++i) U[i + (size_t)nb * i] = 1.0L;
-    if (hasA) {
+    if (hasA && keo_ok) {
       const double *Q = K + (size_t)evr::kQ * nb * nb;
       std::vector<long double> q((size_t)nb * nb);
-      double qmax = 0.0;
-      for (int i = 0; i < nb * nb; ++i) qmax = std::max(qmax, std::fabs(Q[i]));
       for (int i = 0; i < nb; ++i)
-        for (int j = 0; j < nb; ++j) {
-          if (std::fabs(Q[i + nb * j] - Q[j + nb * i]) > 1e-13 * qmax) return EVR_OK;
-          q[i + (size_t)nb * j] = 0.5L * ((long double)Q[i + nb * j] + Q[j + nb * i]);
-        }
+        for (int j = 0; j < nb; ++j) q[i + (size_t)nb * j] = 0.5L * ((long double)Q[i + nb * j] + Q[j + nb * i]);
       jacobi_eig(nb, q, U, lam);
     }
     auto put = [&](int rows, int cols, auto val) {
@@ -752,6 +773,12 @@ int build_hterms(evr_plan *p, const HtInput &h)
     });
     oI[s] = put(nb, nb, [&](int r, int c) { return U[c + (size_t)nb * r]; });
     oO[s] = put(nb, nb, [&](int r, int c) { return U[r + (size_t)nb * c]; });
+    oP[s] = oB[s];
+    oQ[s] = oW[s];
+    if (hasA && keo_ok) {
+      oP[s] = put(nq, nb, [&](int r, int c) { return B[r + (size_t)nq * c]; });
+      oQ[s] = put(nb, nq, [&](int r, int c) { return W[r + (size_t)nb * c]; });
+    }
     // U^T F U
     auto rot = [&](std::vector<long double> F) {
       std::vector<long double> t((size_t)nb * nb, 0.0L), o((size_t)nb * nb, 0.0L);
@@ -801,6 +828,10 @@ int build_hterms(evr_plan *p, const HtInput &h)
 
   // ---- terms
   std::vector<evr::HTerm> ht(p->nterms);
+  std::vector<evr::XTerm> xt(p->nterms);
+  std::vector<int> xcap[2], xrest[2][kNumClasses];  // [grid -> basis, basis -> grid]
+  xcap[0].assign(p->nterms, -1);
+  xcap[1].assign(p->nterms, -1);
   std::vector<evr::HGroup> groups;
   std::vector<double> coef;
   std::map<std::vector<int>, int> coef_of;
@@ -853,12 +884,54 @@ int build_hterms(evr_plan *p, const HtInput &h)
         G.mW[k] = oW[s];
         G.mI[k] = oI[s];
         G.mO[k] = oO[s];
+        G.mP[k] = oP[s];
+        G.mQ[k] = oQ[s];
         G.pw[k] = oO[s] + p->slots[s].nb * p->slots[s].nb - oB[s];
       }
       j += gm1.back() >= 0 ? 2 : 1;
       groups.push_back(G);
     }
     H.ng = (int)groups.size() - H.g0;
+    // basis <-> grid transforms of the term
+    {
+      evr::XTerm &X = xt[t];
+      X.off_nb = td.off_nb;
+      X.off_nq = td.off_nq;
+      X.w = std::fabs(td.w) < 1e-6 ? 0.0 : td.w;
+      X.nbt = td.nbt;
+      X.nqt = td.nqt;
+      X.ng = H.ng;
+      X.g0 = H.g0;
+      X.D = D;
+      X.nvq = X.Pl = X.Ph = X.Rl = X.Rh = 1;
+      int64_t cur = td.nbt;
+      for (int g = 0; g < H.ng; ++g) {
+        const evr::HGroup &G = groups[H.g0 + g];
+        // size before group g is up: a G->B output; after it: a B->G output
+        int &u = ((H.ng - 1 - g) & 1) ? X.uA : X.uB;
+        u = (int)std::max<int64_t>(u, cur);
+        cur = cur / G.nb * G.nq;
+        int &w = (g & 1) ? X.wB : X.wA;
+        w = (int)std::max<int64_t>(w, std::min<int64_t>(cur, INT32_MAX));
+      }
+      X.nvq = (int)std::min<int64_t>(cur, INT32_MAX);
+      X.uA = std::max(X.uA, X.nvq);
+      for (int d = 0; d < D; ++d) {
+        const bool low = X.Pl < 128;
+        X.nlow += low;
+        (low ? X.Pl : X.Ph) *= nq[d];
+        X.nq[d] = nq[d];
+        X.one[d] = nb[d] > 1 ? -1 : (int)p->slots[td.slot[d]].offB;
+        if (nb[d] > 1) (low ? X.Rl : X.Rh) *= nq[d];
+      }
+      if (X.Pl > X.Rl) X.uB = std::max(X.uB, X.Pl * (evr::kXThreads / 64) * evr::kXRows);  // low points of a wave
+      for (int b2g = 0; b2g < 2; ++b2g) {
+        const size_t need = 8 * evr::xform_words(X, b2g);
+        for (int k = 0; k < kXClasses; ++k)
+          if (need <= (size_t)kXLds[k]) xcap[b2g][t] = k;
+        if (xcap[b2g][t] < 0) xrest[b2g][c].push_back((int)t);
+      }
+    }
     // pencil mode: the slowest active mode of three functions
     std::vector<int> act(td.amode, td.amode + td.na);
     H.na = td.na;
@@ -1042,9 +1115,37 @@ int build_hterms(evr_plan *p, const HtInput &h)
   HIP_TRY(p->d_hfac.upload(fac.data(), fac.size(), p->stream));
   HIP_TRY(p->d_hcoef.upload(coef.data(), coef.size(), p->stream));
   HIP_TRY(p->d_horder.upload(order.data(), order.size(), p->stream));
+  // ---- transforms: terms by LDS class, largest grids first
+  for (int b2g = 0; b2g < 2; ++b2g) {
+    std::vector<int> xorder;
+    for (int k = 0; k < kXClasses; ++k) {
+      p->x_off[b2g][k] = (int64_t)xorder.size();
+      for (int64_t t = 0; t < p->nterms; ++t)
+        if (xcap[b2g][t] == k) {
+          xorder.push_back((int)t);
+          p->x_lds[b2g][k] = std::max(p->x_lds[b2g][k], 8 * evr::xform_words(xt[t], b2g));
+        }
+      std::stable_sort(xorder.begin() + p->x_off[b2g][k], xorder.end(),
+                       [&](int a, int b) { return xt[a].nqt > xt[b].nqt; });
+    }
+    p->x_off[b2g][kXClasses] = (int64_t)xorder.size();
+    HIP_TRY(p->d_xorder[b2g].upload(xorder.data(), xorder.size(), p->stream));
+    for (int c = 0; c < kNumClasses; ++c) {
+      std::vector<int> &r = xrest[b2g][c];
+      while (r.size() % 8) r.push_back(-1);
+      p->x_nrest[b2g][c] = (int64_t)r.size();
+      HIP_TRY(p->d_x_rest[b2g][c].upload(r.data(), r.size(), p->stream));
+    }
+  }
+  HIP_TRY(p->d_xt.upload(xt.data(), xt.size(), p->stream));
+  if (!keo_ok) {
+    std::fill(cap.begin(), cap.end(), -1);
+    for (int c = 0; c < kNumClasses; ++c) p->ht_nrest[c] = p->nunits[c];
+  }
   p->ht_on.resize(p->nterms);
   for (int64_t t = 0; t < p->nterms; ++t) p->ht_on[t] = cap[t] >= 0;
-  p->ht = true;
+  p->ht = keo_ok;
+  p->xt = true;
   return EVR_OK;
 }
 
@@ -1108,6 +1209,38 @@ void profile_slot(evr_plan *p, int slot, double flops)
   p->launches[slot] += 1;
 }
 
+// The terms of a basis <-> grid transform that run in register blocks.
+int run_xterms(evr_plan *p, bool b2g, int nvec, const double *X, double *R, double *G, const double *Gin)
+{
+  evr::XArgs a{};
+  a.nvec = nvec;
+  a.terms = (const evr::XTerm EVR_CONST *)p->d_xt.ptr;
+  a.groups = (const evr::HGroup EVR_CONST *)p->d_hg.ptr;
+  a.pool = (evr::ctab)p->d_hpool.ptr;
+  a.pool1 = p->d_bw64.ptr;
+  a.map = p->d_map.ptr;
+  a.rowpos = p->d_rowpos.ptr;
+  a.X = X;
+  a.G = G;
+  a.Gin = Gin;
+  a.R = R;
+  a.gld = p->sum_nq;
+  for (int k = 0; k < kXClasses;) {
+    // classes too small to fill the device share a launch
+    int hi = k + 1;
+    size_t lds = p->x_lds[b2g][k];
+    while (hi < kXClasses && (p->x_off[b2g][hi + 1] - p->x_off[b2g][k]) * nvec <= 8 * (int64_t)p->ncu) {
+      lds = std::max(lds, p->x_lds[b2g][hi]);
+      ++hi;
+    }
+    a.order = (const int EVR_CONST *)(p->d_xorder[b2g].ptr + p->x_off[b2g][k]);
+    const hipError_t e = evr::launch_xform(a, b2g, p->x_off[b2g][hi] - p->x_off[b2g][k], lds, p->stream);
+    if (e != hipSuccess) return fail(EVR_ERR_HIP, std::string("transform kernel: ") + hipGetErrorString(e));
+    k = hi;
+  }
+  return EVR_OK;
+}
+
 // Apply every term class for `nvec` vectors held in X ([nb_packed][nvec]).
 template <typename T>
 int run_terms(evr_plan *p, int mode, int nvec, const T *X, T *R, T *G, const T *Gin, const T *bw,
@@ -1115,7 +1248,7 @@ int run_terms(evr_plan *p, int mode, int nvec, const T *X, T *R, T *G, const T *
 {
   if (!p->one.empty() && !diagKeo && (mode == evr::kModeHpsi || mode == evr::kModeB2G || mode == evr::kModeG2B))
     return run_streamed<T>(p, p->one, mode, nvec, X, R, G, Gin);
-  bool blocks = false;  // the terms in register blocks; the classes keep the rest
+  bool blocks = false, xform = false;  // the terms in register blocks; the classes keep the rest
   if constexpr (sizeof(T) == 8) {
     blocks = p->ht && mode == evr::kModeHpsi;
     if (blocks) {
@@ -1124,14 +1257,23 @@ int run_terms(evr_plan *p, int mode, int nvec, const T *X, T *R, T *G, const T *
       if (rc) return rc;
       if (p->profiling) profile_slot(p, kProfHt, p->flops_ht * nvec);
     }
+    xform = p->xt && !diagKeo && (mode == evr::kModeB2G || mode == evr::kModeG2B);
+    if (xform) {
+      const bool b2g = mode == evr::kModeB2G;
+      const int slot = b2g ? kProfB2g : kProfG2b;
+      if (p->profiling) (void)hipEventRecord(p->ev[2 * slot], p->stream);
+      const int rc = run_xterms(p, b2g, nvec, X, R, G, Gin);
+      if (rc) return rc;
+      if (p->profiling) profile_slot(p, slot, 0.0);
+    }
   }
   for (int c = 0; c < kNumClasses; ++c) {
-    const int64_t units = blocks ? p->ht_nrest[c] : p->nunits[c];
+    const int64_t units = blocks ? p->ht_nrest[c] : (xform ? p->x_nrest[mode == evr::kModeB2G][c] : p->nunits[c]);
     if (units == 0) continue;
     evr::TermParams<T> prm = base_params<T>(p, mode, nvec);
     prm.diagKeo = diagKeo;
     prm.nunits = units;
-    prm.order = blocks ? p->d_ht_rest[c].ptr : p->d_order[c].ptr;
+    prm.order = blocks ? p->d_ht_rest[c].ptr : (xform ? p->d_x_rest[mode == evr::kModeB2G][c].ptr : p->d_order[c].ptr);
     prm.bw = bw;
     prm.keo = keo;
     prm.V = V;
@@ -2497,9 +2639,10 @@ int evr_plan_kernel_stats(evr_plan *p, int max, char *names, double *ms, double 
     if (launches) launches[k] = p->launches[c];
     ++k;
   }
-  for (int c : {kProfAsm, kProfHt}) {
+  for (int c = kProfAsm; c < kProfSlots; ++c) {
+    constexpr const char *kNames[] = {"k_apply_asm", "k_hterm", "k_b2g", "k_g2b"};
     if (p->launches[c] == 0 || k >= max) continue;
-    if (names) snprintf(names + 64 * k, 64, c == kProfAsm ? "k_apply_asm" : "k_hterm");
+    if (names) snprintf(names + 64 * k, 64, "%s", kNames[c - kProfAsm]);
     if (ms) ms[k] = p->ms_acc[c];
     if (flops) flops[k] = p->flops_acc[c];
     if (launches) launches[k] = p->launches[c];

@@ -1,5 +1,5 @@
-"""H|psi> of the Smolyak terms in register blocks against the oracle: every
-group shape of the kernel and the generic one (the 1D laws 1 + 2l functions on
+"""H|psi> and transforms of the Smolyak terms in register blocks against the
+oracle: every group shape of the kernel and the generic one (the 1D laws 1 + 2l functions on
 2 + 2l or 1 + 2l points, 1 + l on 2 + l, 2 + 2l on 3 + 2l; slots up to 19
 functions), terms of one function, terms whose V part runs in slabs (seven
 active modes), one to nine vectors, the kinetic part with and without a
@@ -49,3 +49,28 @@ def test_hterm(evr, oracle_mod, D, L, law, type_, kind, nvec):
     e = np.abs(plan.TabOpPsi(X) - ref).max() / np.abs(ref).max()
     print("D=%d L=%d law %s type %d %s, %d vectors: %.2e" % (D, L, law, type_, kind, nvec, e))
     assert e < TOL64
+
+
+@pytest.mark.parametrize("D,L,law,ncol", [(1, 3, (1, 2, 2, 2), 1), (2, 9, (1, 2, 2, 2), 2), (4, 4, (1, 2, 1, 2), 2),
+                                          (4, 3, (1, 1, 2, 1), 2), (3, 3, (2, 2, 3, 2), 3), (6, 5, (1, 2, 2, 2), 5),
+                                          (7, 7, (1, 2, 2, 2), 1), (9, 4, (1, 2, 2, 2), 2), (12, 3, (1, 2, 2, 2), 1),
+                                          (12, 2, (1, 2, 1, 2), 3)])
+def test_transforms(evr, oracle_mod, D, L, law, ncol):
+    """Basis -> grid and the weighted grid -> basis in register blocks: few and
+    many one-function modes, their points below and above the low part of 128,
+    terms whose reduced grid stays with the term kernels (seven modes)."""
+    s = oracle_mod.SG4(D, L, L, *law)
+    b = evr.Basis.sg4(D, L, L, *law)
+    # a q-linear G: the H|psi> tables of such a plan are rotated, these are not
+    plan = evr.Plan(b, type=10, G0=np.eye(D), Ga=np.full(D ** 3, 0.01), max_nvec=ncol)
+    rng = np.random.RandomState(D * 10 + L)
+    X = np.asfortranarray(rng.randn(b.nb_packed, ncol))
+    G = plan.BasisRep_TO_GridRep_n(X)
+    for c in range(ncol):
+        ref = s.b2g(X[:, c])
+        assert np.abs(G[:, c] - ref).max() / np.abs(ref).max() < TOL64
+    Gr = np.asfortranarray(rng.randn(b.sum_nq, ncol))
+    Y = plan.GridRep_TO_BasisRep_n(Gr)
+    for c in range(ncol):
+        ref = s.g2b(Gr[:, c])
+        assert np.abs(Y[:, c] - ref).max() / np.abs(ref).max() < TOL64
