@@ -116,6 +116,27 @@ struct HArgs {
   double *R;
 };
 
+// Grid form of type 10 with G, J, s per point, one term per workgroup
+// (evr_gkterm.hip); psi_G, out in T, tables FP64.
+template <typename T>
+struct GkArgs {
+  int k;                   // vectors
+  int trans;               // the weighted transpose
+  const int *order;        // terms of the workgroups (-1 = padding)
+  const TermDev *terms;
+  const SlotDev *slots;
+  const double *D1, *ain, *J, *GG, *s, *V, *wq;
+  const T *G;
+  T *F;
+  int64_t sum_nq;
+};
+// points a thread holds, their D derivatives in registers: with 4 the D=6 kernel
+// spills 164 registers of its 128 (726 us for the H|psi> of D=6 L=5 with 8
+// vectors, 285 us with 2)
+constexpr int kGkPoints = 2;
+template <typename T>
+hipError_t launch_gk_term(const GkArgs<T> &a, int D, int64_t units, int nt, size_t lds, hipStream_t s);
+
 // threads and LDS words of a transform workgroup; high r points a wave of the
 // G->B contraction takes at a time
 constexpr int kXThreads = 256;

@@ -102,6 +102,9 @@ constexpr int kKiB = 1024;
 constexpr HtClass kHtClasses[] = {{0, 160 * kKiB, 1024}, {0, 80 * kKiB, 512}, {0, 53 * kKiB, 320}, {0, 40 * kKiB, 256},
                                   {1, 40 * kKiB, 256},   {2, 40 * kKiB, 256}, {3, 40 * kKiB, 256}};
 constexpr int kHtCaps = sizeof(kHtClasses) / sizeof(kHtClasses[0]);
+// threads of the grid-form workgroups
+constexpr int kGkThreads[] = {1024, 512, 256, 128};
+constexpr int kGkCaps = sizeof(kGkThreads) / sizeof(kGkThreads[0]);
 // LDS classes of the transform workgroups (256 threads): 1, 2, 4, 8 per CU
 constexpr int kXLds[] = {160 * kKiB, 80 * kKiB, 40 * kKiB, 20 * kKiB};
 constexpr int kXClasses = sizeof(kXLds) / sizeof(kXLds[0]);
@@ -150,6 +153,12 @@ struct evr_plan {
   int64_t n_gitems = 0;
   DevBuf<double> d_GG, d_Jg, d_Sg, d_Gg, d_Pg, d_Fg;
   DevBuf<int2> d_gitems;
+  // type 10 in one pass per term (evr_gkterm.hip) when every term grid fits a
+  // workgroup: work list by thread count
+  bool gk_term = false;
+  DevBuf<int> d_gkorder;
+  int64_t gk_off[kGkCaps + 1] = {};
+  size_t gk_lds[kGkCaps] = {};
   // hermitian grid form: quadrature weight per point, w / (J s), and the term
   // rows of the transposed sequence
   DevBuf<double> d_Wq, d_As, d_R2, d_F2w, d_F1w;
@@ -247,6 +256,7 @@ struct evr_plan {
       d_x_rest[0][c].release();
       d_x_rest[1][c].release();
     }
+    d_gkorder.release();
     d_xt.release(); d_xorder[0].release(); d_xorder[1].release();
     d_Wq.release(); d_As.release(); d_R2.release(); d_F2w.release(); d_F1w.release();
     for (auto &e : ev)
@@ -1475,9 +1485,45 @@ hipError_t launch_items(int c, const evr::TermParams<double> &prm, int64_t nitem
   }
 }
 
+// psi_G -> the grid form of type 10 on every term (trans: its weighted
+// transpose), one launch per thread count; counts with too few workgroups to
+// fill the device share one.
+template <typename T>
+int run_gk_terms(evr_plan *p, int k, int trans, const T *G, T *F)
+{
+  evr::GkArgs<T> a{};
+  a.k = k;
+  a.trans = trans;
+  a.terms = p->d_terms.ptr;
+  a.slots = p->d_slots.ptr;
+  a.D1 = p->d_D1.ptr;
+  a.ain = trans ? p->d_As.ptr : p->d_Sg.ptr;
+  a.J = p->d_Jg.ptr;
+  a.GG = p->d_GG.ptr;
+  a.s = p->d_Sg.ptr;
+  a.V = p->d_V.ptr;
+  a.wq = trans ? p->d_Wq.ptr : nullptr;
+  a.G = G;
+  a.F = F;
+  a.sum_nq = p->sum_nq;
+  for (int lo = 0; lo < kGkCaps;) {
+    int hi = lo + 1;
+    size_t lds = p->gk_lds[lo];
+    while (hi < kGkCaps && (p->gk_off[hi + 1] - p->gk_off[lo]) * k <= 4 * (int64_t)p->ncu) {
+      lds = std::max(lds, p->gk_lds[hi]);
+      ++hi;
+    }
+    a.order = p->d_gkorder.ptr + p->gk_off[lo];
+    const hipError_t e = evr::launch_gk_term<T>(a, p->D, p->gk_off[hi] - p->gk_off[lo], kGkThreads[lo], lds, p->stream);
+    if (e != hipSuccess) return fail(EVR_ERR_HIP, std::string("grid form: ") + hipGetErrorString(e));
+    lo = hi;
+  }
+  return EVR_OK;
+}
+
 // H|psi> of a plan with G, J, s (or F2, F1) per grid point into dh (device,
-// nb_packed x nvec): B->G, the reference's grid form of every term
-// (k_gk_deriv, k_gk_combine, k_gk_out or k_t1_out, V included), then the
+// nb_packed x nvec): B->G, the reference's grid form of every term (k_gk_term,
+// or k_gk_deriv, k_gk_combine, k_gk_out or k_t1_out, V included), then the
 // weighted G->B and the deterministic scatter, gvec vectors at a time.  T is
 // the precision of the transforms and of the grid columns (FP32 keeps the
 // tables and the grid arithmetic in FP64; the work grids hold floats).
@@ -1505,23 +1551,28 @@ int keo_grid_hpsi(evr_plan *p, int nvec, const double *dpsi, double *dh)
     }
     if (rc) return rc;
     const bool t1 = p->grid_type == 1;
-    hipLaunchKernelGGL(evr::k_gk_deriv<T>, dim3((unsigned)p->n_gitems), dim3(256), 0, p->stream, D,
-                       p->d_terms.ptr, p->d_slots.ptr, p->d_D1.ptr, p->d_gitems.ptr,
-                       t1 ? nullptr : p->d_Sg.ptr, Gg, nq, k, Pg, 0);
-    HIP_TRY(hipGetLastError());
-    if (t1) {
-      hipLaunchKernelGGL(evr::k_t1_out<T>, dim3((unsigned)p->n_gitems), dim3(256), 0, p->stream, D,
-                         p->d_terms.ptr, p->d_slots.ptr, p->d_D1.ptr, p->d_D2.ptr, p->d_gitems.ptr,
-                         p->d_F2g.ptr, p->d_F1g.ptr, p->d_V.ptr, Gg, Pg, nq, k, Fg);
-      HIP_TRY(hipGetLastError());
+    if (p->gk_term) {
+      rc = run_gk_terms<T>(p, k, 0, Gg, Fg);
+      if (rc) return rc;
     } else {
-      hipLaunchKernelGGL(evr::k_gk_combine<T>, dim3(blocks_for(nq)), dim3(256), 0, p->stream, D, nq, k,
-                         p->d_GG.ptr, p->d_Jg.ptr, Pg, 0);
+      hipLaunchKernelGGL(evr::k_gk_deriv<T>, dim3((unsigned)p->n_gitems), dim3(256), 0, p->stream, D,
+                         p->d_terms.ptr, p->d_slots.ptr, p->d_D1.ptr, p->d_gitems.ptr,
+                         t1 ? nullptr : p->d_Sg.ptr, Gg, nq, k, Pg, 0);
       HIP_TRY(hipGetLastError());
-      hipLaunchKernelGGL(evr::k_gk_out<T>, dim3((unsigned)p->n_gitems), dim3(256), 0, p->stream, D,
-                         p->d_terms.ptr, p->d_slots.ptr, p->d_D1.ptr, p->d_gitems.ptr, p->d_Jg.ptr,
-                         p->d_Sg.ptr, p->d_V.ptr, Gg, Pg, nq, k, Fg, (const double *)nullptr);
-      HIP_TRY(hipGetLastError());
+      if (t1) {
+        hipLaunchKernelGGL(evr::k_t1_out<T>, dim3((unsigned)p->n_gitems), dim3(256), 0, p->stream, D,
+                           p->d_terms.ptr, p->d_slots.ptr, p->d_D1.ptr, p->d_D2.ptr, p->d_gitems.ptr,
+                           p->d_F2g.ptr, p->d_F1g.ptr, p->d_V.ptr, Gg, Pg, nq, k, Fg);
+        HIP_TRY(hipGetLastError());
+      } else {
+        hipLaunchKernelGGL(evr::k_gk_combine<T>, dim3(blocks_for(nq)), dim3(256), 0, p->stream, D, nq, k,
+                           p->d_GG.ptr, p->d_Jg.ptr, Pg, 0);
+        HIP_TRY(hipGetLastError());
+        hipLaunchKernelGGL(evr::k_gk_out<T>, dim3((unsigned)p->n_gitems), dim3(256), 0, p->stream, D,
+                           p->d_terms.ptr, p->d_slots.ptr, p->d_D1.ptr, p->d_gitems.ptr, p->d_Jg.ptr,
+                           p->d_Sg.ptr, p->d_V.ptr, Gg, Pg, nq, k, Fg, (const double *)nullptr);
+        HIP_TRY(hipGetLastError());
+      }
     }
     rc = run_terms<T>(p, evr::kModeG2B, k, nullptr, R, nullptr, Fg, bw, keo, nullptr);
     if (rc) return rc;
@@ -1531,17 +1582,22 @@ int keo_grid_hpsi(evr_plan *p, int nvec, const double *dpsi, double *dh)
       // and the weighted G->B: d_i^T on (w / (J s)) psi_G, J sum_i G_ji,
       // -1/2 (s / w) sum_j d_j^T; the rows of H and H^T are then averaged
       T *R2 = reinterpret_cast<T *>(p->d_R2.ptr);
-      hipLaunchKernelGGL(evr::k_gk_deriv<T>, dim3((unsigned)p->n_gitems), dim3(256), 0, p->stream, D,
-                         p->d_terms.ptr, p->d_slots.ptr, p->d_D1.ptr, p->d_gitems.ptr, p->d_As.ptr, Gg, nq, k,
-                         Pg, 1);
-      HIP_TRY(hipGetLastError());
-      hipLaunchKernelGGL(evr::k_gk_combine<T>, dim3(blocks_for(nq)), dim3(256), 0, p->stream, D, nq, k,
-                         p->d_GG.ptr, p->d_Jg.ptr, Pg, 1);
-      HIP_TRY(hipGetLastError());
-      hipLaunchKernelGGL(evr::k_gk_out<T>, dim3((unsigned)p->n_gitems), dim3(256), 0, p->stream, D,
-                         p->d_terms.ptr, p->d_slots.ptr, p->d_D1.ptr, p->d_gitems.ptr, p->d_Jg.ptr,
-                         p->d_Sg.ptr, p->d_V.ptr, Gg, Pg, nq, k, Fg, (const double *)p->d_Wq.ptr);
-      HIP_TRY(hipGetLastError());
+      if (p->gk_term) {
+        rc = run_gk_terms<T>(p, k, 1, Gg, Fg);
+        if (rc) return rc;
+      } else {
+        hipLaunchKernelGGL(evr::k_gk_deriv<T>, dim3((unsigned)p->n_gitems), dim3(256), 0, p->stream, D,
+                           p->d_terms.ptr, p->d_slots.ptr, p->d_D1.ptr, p->d_gitems.ptr, p->d_As.ptr, Gg, nq, k,
+                           Pg, 1);
+        HIP_TRY(hipGetLastError());
+        hipLaunchKernelGGL(evr::k_gk_combine<T>, dim3(blocks_for(nq)), dim3(256), 0, p->stream, D, nq, k,
+                           p->d_GG.ptr, p->d_Jg.ptr, Pg, 1);
+        HIP_TRY(hipGetLastError());
+        hipLaunchKernelGGL(evr::k_gk_out<T>, dim3((unsigned)p->n_gitems), dim3(256), 0, p->stream, D,
+                           p->d_terms.ptr, p->d_slots.ptr, p->d_D1.ptr, p->d_gitems.ptr, p->d_Jg.ptr,
+                           p->d_Sg.ptr, p->d_V.ptr, Gg, Pg, nq, k, Fg, (const double *)p->d_Wq.ptr);
+        HIP_TRY(hipGetLastError());
+      }
       rc = run_terms<T>(p, evr::kModeG2B, k, nullptr, R2, nullptr, Fg, bw, keo, nullptr);
       if (rc) return rc;
       const int64_t nr = p->nrows * k;
@@ -1604,10 +1660,44 @@ int grid_form_buffers(evr_plan *p)
   const int64_t nq = p->sum_nq;
   int rc = grid_items(p);
   if (rc) return rc;
-  // (D + 2) x sum_nq doubles per vector
-  p->gvec = (int)std::max<int64_t>(1, std::min<int64_t>(p->max_nvec, (int64_t)(8e9 / (8.0 * (D + 2) * nq))));
+  if (p->type == 10) {
+    std::vector<int> order, cap(p->nterms, -1);
+    std::vector<size_t> lds(p->nterms, 0);
+    p->gk_term = true;
+    for (int64_t t = 0; t < p->nterms; ++t) {
+      const evr::TermDev &td = p->terms[t];
+      lds[t] = td.nqt;
+      bool wide = false;  // beyond the kernel's 5-bit digits
+      for (int d = 0; d < D; ++d) {
+        const int nq1 = p->slots[td.slot[d]].nq;
+        lds[t] += nq1 * nq1;
+        wide = wide || nq1 > 32;
+      }
+      lds[t] *= 8;
+      for (int k = 0; k < kGkCaps; ++k)
+        if (td.nqt <= kGkThreads[k] * evr::kGkPoints) cap[t] = k;
+      if (cap[t] < 0 || wide || lds[t] > kLdsLimit) p->gk_term = false;
+    }
+    for (int k = 0; k < kGkCaps && p->gk_term; ++k) {
+      std::vector<int> ids;
+      for (int64_t t = 0; t < p->nterms; ++t)
+        if (cap[t] == k) {
+          ids.push_back((int)t);
+          p->gk_lds[k] = std::max(p->gk_lds[k], lds[t]);
+        }
+      std::stable_sort(ids.begin(), ids.end(), [&](int a, int b) { return p->terms[a].nqt > p->terms[b].nqt; });
+      while (ids.size() % 8) ids.push_back(-1);
+      p->gk_off[k] = (int64_t)order.size();
+      order.insert(order.end(), ids.begin(), ids.end());
+    }
+    p->gk_off[kGkCaps] = (int64_t)order.size();
+    if (p->gk_term) HIP_TRY(p->d_gkorder.upload(order.data(), order.size(), p->stream));
+  }
+  // (D + 2) x sum_nq doubles per vector (two without the derivative columns)
+  const int cols = p->gk_term ? 2 : D + 2;
+  p->gvec = (int)std::max<int64_t>(1, std::min<int64_t>(p->max_nvec, (int64_t)(8e9 / (8.0 * cols * nq))));
   HIP_TRY(p->d_Gg.alloc((size_t)nq * p->gvec));
-  HIP_TRY(p->d_Pg.alloc((size_t)nq * D * p->gvec));
+  if (!p->gk_term) HIP_TRY(p->d_Pg.alloc((size_t)nq * D * p->gvec));
   HIP_TRY(p->d_Fg.alloc((size_t)nq * p->gvec));
   return EVR_OK;
 }

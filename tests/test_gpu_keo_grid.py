@@ -111,3 +111,34 @@ def test_keo_grid_hermitian(evr, oracle_mod):
     print("hermitian G per point: %.3e, FP32 %.3e, diagonal %.3e (asymmetry of H %.2e)" % (err, err32, errd, asym))
     assert asym > 1e-6
     assert err < 1e-12 and errd < 1e-12 and err32 < 2e-5
+
+
+@pytest.mark.parametrize("D,L,law,nvec,herm", [
+    (1, 6, (1, 2, 2, 2), 3, True), (2, 7, (1, 2, 1, 2), 9, False), (5, 5, (1, 2, 2, 2), 1, True),
+    (7, 3, (1, 2, 2, 2), 2, True), (9, 2, (1, 1, 2, 1), 3, False), (12, 2, (1, 2, 2, 2), 1, False),
+    (3, 3, (1, 8, 4, 8), 2, True),    # a term of 1728 points, two per thread
+    (3, 3, (1, 8, 6, 8), 2, True)])   # a term of 2744 points: the three global passes
+def test_keo_grid_terms(evr, oracle_mod, D, L, law, nvec, herm):
+    """One workgroup per term and vector, from term grids of a few points to
+    two points per thread, and the global passes of larger ones: H|psi> and its
+    hermitian form in FP64 and FP32 against the oracle."""
+    s = oracle_mod.SG4(D, L, L, *law)
+    b = evr.Basis.sg4(D, L, L, *law)
+    q = s.grid()
+    Gq, J, sq = tabulated_keo(q, 40 + D)
+    V = 0.5 * (q ** 2).sum(1) + 0.05 * q[:, 0] ** 3
+    op = oracle_mod.Op(10, V=V, Jac=J, s=sq, Gq=Gq)
+    X = evr.hamiltonian.test_vectors(s.nb_packed, nvec, D)
+    for h in ([False, True] if herm else [False]):
+        if h:
+            M = s.oppsi(op, np.eye(s.nb_packed))
+            ref = 0.5 * (M @ X + M.T @ X)
+        else:
+            ref = s.oppsi(op, X)
+        plan = evr.Plan(b, type=10, V=V, G0=np.eye(D), max_nvec=nvec, hermitian=h)
+        plan.set_keo_grid(Gq, J, sq)
+        err = relerr(plan.TabOpPsi(X), ref)
+        err32 = relerr(plan.TabOpPsi(X, flags=evr.FP32), ref)
+        print("D=%d L=%d law %s hermitian %d: %.3e, FP32 %.3e" % (D, L, law, h, err, err32))
+        assert err < 1e-12
+        assert err32 < 2e-5
