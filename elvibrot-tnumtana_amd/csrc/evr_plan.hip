@@ -2,6 +2,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -19,6 +20,7 @@
 #include "evr_setup.hpp"
 #include "evr_term.hip"
 #include "evr_stream.hip"
+#include "evr_dpterm.hpp"
 
 namespace {
 
@@ -173,6 +175,11 @@ struct evr_plan {
   int64_t big_nq = 0;
   int big_k = 0;
   DevBuf<double> d_big;
+  // their FP64 H|psi> in three passes (evr_dpterm.hip): the modes' matrices of
+  // every term of `big` or `one`, in that order
+  bool dp_pass = false, dp_coupled = false, dp_own = false;
+  std::vector<std::array<evr::DpMode, 4>> dp_terms;
+  DevBuf<double> d_dptab, d_dpC;
   std::vector<double> hC, hF1;  // host copies of the KEO coefficients (kernel convention)
   DevBuf<int> d_map, d_rowpos;
   // reduction segments: rows seg[s] .. seg[s+1]-1 of R; the segments of packed
@@ -248,6 +255,7 @@ struct evr_plan {
     for (int c = 0; c < kNumClasses; ++c) d_order[c].release();
     d_X.release(); d_R.release(); d_psi.release(); d_hpsi.release(); d_G.release();
     d_A64.release(); d_A32.release(); d_asm_items.release(); d_D1.release(); d_D2.release();
+    d_dptab.release(); d_dpC.release();
     d_GG.release(); d_Jg.release(); d_Sg.release(); d_Gg.release(); d_Pg.release(); d_Fg.release();
     d_F2g.release(); d_F1g.release(); d_gitems.release(); d_dp_perm.release(); d_big.release();
     d_ht.release(); d_hg.release(); d_hpool.release(); d_hfac.release(); d_hcoef.release(); d_horder.release();
@@ -483,6 +491,168 @@ int apply_classes(evr_plan *p)
   return EVR_OK;
 }
 
+// FP64 H|psi> of one streamed term, k vectors from c0 on, in the three passes
+// of evr_dpterm.hip on the plan stream.
+int run_dp_term(evr_plan *p, const std::array<evr::DpMode, 4> &m, const evr::TermDev &td, int nvec, int c0, int k,
+                const double *X, double *R)
+{
+  const int D = p->D, na = evr::dp_first(D);
+  evr::DpArgs a{};
+  a.k = k;
+  a.nvec = nvec;
+  a.c0 = c0;
+  a.coupled = p->dp_coupled;
+  a.own = p->dp_own;
+  a.hasA = p->hasA;
+  a.tab = p->d_dptab.ptr;
+  a.C = (evr::ctab)p->d_dpC.ptr;
+  a.A = (evr::ctab)p->d_coefA.ptr;
+  a.x = p->d_x.ptr;
+  for (int d = 0; d < D; ++d) {
+    a.m[d] = m[d];
+    a.offX[d] = (int)p->slots[td.slot[d]].offX;
+  }
+  a.V = p->hasV ? p->d_V.ptr + td.off_nq : nullptr;
+  a.X = X;
+  a.map = p->d_map.ptr + td.off_nb;
+  const int64_t S = p->big_nq * p->big_k;
+  for (int i = 0; i < 4; ++i) a.in[i] = p->d_big.ptr + i * S;
+  for (int i = 0; i < 3; ++i) a.out[i] = p->d_big.ptr + (4 + i) * S;
+  a.R = R;
+  a.rowpos = p->d_rowpos.ptr + td.off_nb;
+  a.w = td.w;
+  const bool two = na == 2, two_last = D - na == 2;
+  int64_t nA = 1, nbA = 1, nbB = 1;
+  for (int d = 0; d < D; ++d) {
+    if (d < na) {
+      nA *= m[d].nq;
+      nbA *= m[d].nb;
+    } else {
+      nbB *= m[d].nb;
+    }
+  }
+  const evr::DpMode &u0 = m[0], &v0 = m[na - 1], &u1 = m[na], &v1 = m[D - 1];
+  auto chunks = [](int n) { return (n + evr::kDpOut - 1) / evr::kDpOut; };
+  auto blocks = [](int64_t n) { return (int)((n + evr::kDpPencils - 1) / evr::kDpPencils); };
+  for (int pass = 0; pass < 3; ++pass) {
+    // words of a column, pencils of a column and chunks of the widest step
+    const int words = pass == 0 ? (int)nbA + (two ? u0.nq * v0.nb : 0)
+                          : pass == 1 ? 2 * (two_last ? u1.nq : 1) * v1.nq : (two ? 2 : 1) * (int)nA;
+    const int pens = pass == 1 ? (two_last ? u1.nq : 1) : (two ? std::max(u0.nq, v0.nb) : 1);  // per column, at most
+    const int och = pass == 1 ? std::max(chunks(v1.nq), two_last ? chunks(u1.nq) : 1)
+                              : std::max(chunks(v0.nq), chunks(u0.nq));
+    const int vch = chunks(pass == 1 ? v1.nq : v0.nb);
+    a.ncols = (int)(pass == 1 ? nA * k : nbB * k);
+    // The columns of a tile: the most (64 at most, a line of LDS per point) that
+    // let two workgroups share a CU's LDS and give every CU a tile (17 x 23 x 14,
+    // 5 vectors: 52 us against 68 us with at least 8 columns in 9 tiles); in the
+    // second and third pass a wave holds one item.
+    int cbs = 6;
+    auto fits = [&](int c) {
+      if (pass > 0 && blocks((int64_t)pens << c) * vch > evr::kDpWaves) return false;
+      return ((size_t)words << c) * 8 <= (size_t)80 * kKiB && (a.ncols >> c) >= p->ncu;
+    };
+    while (cbs > 0 && !fits(cbs)) --cbs;
+    a.cbs = cbs;
+    a.ntiles = (a.ncols + (1 << cbs) - 1) >> cbs;
+    const int pb = blocks((int64_t)pens << cbs);
+    const int waves = std::min(pass == 0 ? 8 : evr::kDpWaves, pb * och);
+    const hipError_t e = evr::launch_dp_pass(a, D, pass, 64 * waves, ((size_t)words << cbs) * 8, p->stream);
+    if (e != hipSuccess) return fail(EVR_ERR_HIP, std::string("streamed term pass: ") + hipGetErrorString(e));
+  }
+  return EVR_OK;
+}
+
+// Matrices of the three-pass terms from the slots' 1D matrices and the KEO
+// coefficients.  Terms of two to four modes; the hermitian form of a KEO needs
+// the transposed sequence of the mode-by-mode passes.
+int build_dp_terms(evr_plan *p, const std::vector<double> &bw, const std::vector<double> &d1,
+                   const std::vector<double> &d2)
+{
+  const int D = p->D;
+  const std::vector<int64_t> &list = p->one.empty() ? p->big : p->one;
+  if (list.empty() || D < 2 || D > 4 || (p->hermitian && p->hasKeo)) return EVR_OK;
+  const std::vector<double> &C = p->hC;
+  std::vector<double> Cx(D * D, 0.0), kd(D, 0.0);  // of the cross terms, of D1 D1 or D2
+  bool off = p->hasA;
+  for (int i = 0; i < D; ++i)
+    for (int j = 0; j < D; ++j) off = off || (i != j && C[i * D + j] != 0.0);
+  if (p->type == 10) {
+    if (off) Cx = C;
+    else
+      for (int i = 0; i < D; ++i) kd[i] = C[i * D + i];
+    p->dp_own = !off;
+  } else if (p->type == 1) {
+    // f_ij d_j d_i psi: the bracket of mode j takes P_i
+    for (int i = 0; i < D; ++i)
+      for (int j = 0; j < D; ++j)
+        if (i != j) Cx[j * D + i] = C[i * D + j];
+    for (int i = 0; i < D; ++i) kd[i] = C[i * D + i];
+    p->dp_own = true;
+  } else {
+    off = false;
+  }
+  p->dp_coupled = off;
+  std::vector<double> tab;
+  auto put = [&](int nin, int nout, auto val) {
+    const int o = (int)tab.size(), ld = evr::dp_pad(nout);
+    for (int i = 0; i < (nin + 3) / 4 * 4; ++i)
+      for (int j = 0; j < ld; ++j) tab.push_back(i < nin && j < nout ? val(j, i) : 0.0);
+    return o;
+  };
+  std::vector<std::pair<int, evr::DpMode>> done;  // by slot
+  for (int64_t t : list) {
+    std::array<evr::DpMode, 4> ms{};
+    for (int d = 0; d < D; ++d) {
+      const int s = p->terms[t].slot[d];
+      size_t k = 0;
+      while (k < done.size() && done[k].first != s) ++k;
+      if (k == done.size()) {
+        const evr::SlotDev &sd = p->slots[s];
+        const int nb = sd.nb, nq = sd.nq;
+        const double *B = bw.data() + sd.offB, *W = bw.data() + sd.offW, *E1 = d1.data() + sd.offD1,
+                     *E2 = d2.data() + sd.offD1;
+        const double f1 = p->hasF1 ? p->hF1[d] : 0.0;
+        std::vector<double> DB((size_t)nq * nb), KB((size_t)nq * nb);
+        auto mul = [&](const double *E, const double *M, std::vector<double> &out, double f, bool add) {
+          for (int b = 0; b < nb; ++b)
+            for (int q = 0; q < nq; ++q) {
+              double v = 0.0;
+              for (int r = 0; r < nq; ++r) v += E[q + (size_t)nq * r] * M[r + (size_t)nq * b];
+              out[q + (size_t)nq * b] = (add ? out[q + (size_t)nq * b] : 0.0) + f * v;
+            }
+        };
+        mul(E1, B, DB, 1.0, false);
+        if (p->type == 1) {
+          mul(E2, B, KB, kd[d], false);
+          if (f1 != 0.0) mul(E1, B, KB, f1, true);
+        } else {
+          mul(E1, DB.data(), KB, kd[d], false);
+        }
+        evr::DpMode m{};
+        m.nb = nb;
+        m.nq = nq;
+        m.B = put(nb, nq, [&](int q, int b) { return B[q + (size_t)nq * b]; });
+        m.DB = put(nb, nq, [&](int q, int b) { return DB[q + (size_t)nq * b]; });
+        m.KB = put(nb, nq, [&](int q, int b) { return KB[q + (size_t)nq * b]; });
+        m.W = put(nq, nb, [&](int b, int q) { return W[b + (size_t)nb * q]; });
+        m.WD = put(nq, nb, [&](int b, int q) {
+          double v = 0.0;
+          for (int r = 0; r < nq; ++r) v += W[b + (size_t)nb * r] * E1[r + (size_t)nq * q];
+          return v;
+        });
+        done.push_back({s, m});
+      }
+      ms[d] = done[k].second;
+    }
+    p->dp_terms.push_back(ms);
+  }
+  HIP_TRY(p->d_dptab.upload(tab.data(), tab.size(), p->stream));
+  HIP_TRY(p->d_dpC.upload(Cx.data(), Cx.size(), p->stream));
+  p->dp_pass = true;
+  return EVR_OK;
+}
+
 // The streamed terms of a run_terms call (evr_stream.hip), one term and up to
 // big_k vectors at a time: H|psi> reads X and writes the term rows of R, B2G
 // reads X and writes the grid columns of G, G2B reads the grid columns of Gin
@@ -497,7 +667,8 @@ int run_streamed(evr_plan *p, const std::vector<int64_t> &list, int mode, int nv
   T *b_in = base, *b_g = base + S, *b_a = base + 2 * S, *b_b = base + 3 * S, *b_acc = base + 4 * S,
     *b_y0 = base + 5 * S, *b_y1 = base + 6 * S, *b_P = base + 7 * S;
   auto blocks = [](int64_t n) { return (unsigned)std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, 65536)); };
-  for (int64_t t : list) {
+  for (size_t n = 0; n < list.size(); ++n) {
+    const int64_t t = list[n];
     const evr::TermDev &td = p->terms[t];
     int nb[evr::kMaxDev], nq[evr::kMaxDev];
     const evr::SlotDev *sl[evr::kMaxDev];
@@ -511,6 +682,12 @@ int run_streamed(evr_plan *p, const std::vector<int64_t> &list, int mode, int nv
       const int k = std::min(p->big_k, nvec - c0);
       const int64_t nbk = (int64_t)td.nbt * k, nqk = (int64_t)td.nqt * k;
       if (nqk >= INT32_MAX) return fail(EVR_ERR_SIZE, "streamed term grid too large for one pass");
+      if constexpr (sizeof(T) == 8)
+        if (p->dp_pass && mode == evr::kModeHpsi) {
+          const int rc = run_dp_term(p, p->dp_terms[n], td, nvec, c0, k, X, R);
+          if (rc) return rc;
+          continue;
+        }
       hipError_t e = hipSuccess;
       auto pass = [&](const T *in, T *out, const double *M, int ld, int trans, int64_t L, int nin, int nout,
                       int64_t Rr, int accum = 0, double scale = 1.0) {
@@ -2184,6 +2361,8 @@ int evr_plan_create(const evr_basis_desc *bd, const evr_op_desc *op, int max_nve
     if (rc) return rc;
     const int rch = build_hterms(p.get(), HtInput{bw, keo, cC, cA, cF1, sets, D, nlev});
     if (rch) return rch;
+    const int rcd = build_dp_terms(p.get(), bw, d1, d2);
+    if (rcd) return rcd;
   }
 
   // ---- deterministic scatter: the term rows of packed function pk, in

@@ -9,6 +9,9 @@
 //                   F2/F1 derivative sums or the type-10 -1/2 d_i G_ji(q) d_j
 //   grid -> basis   GDP_TO_BDP_OF_SmolyakRep (BGSG4:2497-2581)
 // with the grid derivative of DerivOp_TO_RDP_OF_SmolaykRep (BGSG4:2690-2795).
+// (FP64 H|psi> of two to four modes runs in three passes instead,
+// evr_dpterm.hip; these kernels keep FP32, the transforms, the hermitian form
+// and one mode or more than four.)
 // Tensors are [point or function][vector]: the vectors of the chunk fastest,
 // then mode 0, mode 1, ... (the term's own basis and grid orders).
 #pragma once
