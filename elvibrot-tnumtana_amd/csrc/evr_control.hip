@@ -332,9 +332,9 @@ extern "C" int evr_control_gradient(evr_plan *H, evr_plan *mu, const evr_control
     HTRY(ST.alloc(nblk * (int64_t)kseg * std::min(ck, N)));
     // g = dJ/dpsi(T) = 2 <phi1|psi(T)> phi1
     {
-      std::vector<cplx> c(nf), zero(nf, 0.0);
+      std::vector<cplx> c(nf);
       for (int f = 0; f < nf; ++f) c[f] = 2.0 * ov[f];
-      RTRY(P.comb(PHI.p, 0, 1, c, &zero, G.p));
+      RTRY(P.comb(PHI.p, 0, 1, c, nullptr, G.p));
     }
     for (int seg = nck - 1; seg >= 0; --seg) {
       const int s0 = seg * ck, s1 = std::min(N, s0 + ck);

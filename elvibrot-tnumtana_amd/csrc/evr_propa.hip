@@ -1096,12 +1096,12 @@ static int propagate_impl(OpRef H, OpRef mu, const evr_propa_opts *o, int nwp, d
       std::vector<cplx> nn;
       RTRY(P.dots(PSI.p, 0, 1, PSI.p, nn));
       std::vector<double> nu(nwp);
-      std::vector<cplx> a(nwp), zero(nwp, 0.0), one(nwp, 1.0);
+      std::vector<cplx> a(nwp), one(nwp, 1.0);  // no 0 x Y: Q starts unset
       for (int w = 0; w < nwp; ++w) {
         nu[w] = std::sqrt(std::max(nn[w].real(), 0.0));
         a[w] = nu[w] > 0.0 ? 1.0 / nu[w] : 0.0;
       }
-      RTRY(P.comb(PSI.p, 0, 1, a, &zero, Q.p));
+      RTRY(P.comb(PSI.p, 0, 1, a, nullptr, Q.p));
       std::vector<std::vector<double>> al(nwp), be(nwp, std::vector<double>(1, 0.0));
       std::vector<double> e0(nwp, 0.0);
       std::vector<std::vector<cplx>> U(nwp);
@@ -1142,7 +1142,7 @@ static int propagate_impl(OpRef H, OpRef mu, const evr_propa_opts *o, int nwp, d
           be[w].push_back(b);
           ib[w] = b > 0.0 ? 1.0 / b : 0.0;
         }
-        RTRY(P.comb(HW.p, 0, 1, ib, &zero, Q.p + nblk * (k + 1)));
+        RTRY(P.comb(HW.p, 0, 1, ib, nullptr, Q.p + nblk * (k + 1)));
       }
       max_order = std::max(max_order, n);
       // psi = nu exp(-i E0 dt) sum_k u_k q_k

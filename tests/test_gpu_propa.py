@@ -104,6 +104,23 @@ def test_sil_sg4(evr, sg4_case):
     assert abs(info.max_order - ors) <= 1
 
 
+def test_sil_fresh_memory(evr, sg4_case):
+    """The Krylov block takes whatever device memory holds: memory full of NaN
+    (freed just before) changes nothing."""
+    from conftest import DeviceBuffer
+    c = sg4_case
+    psi = rand_psi(c["nb"], 2, 3)
+    ex = propa.exact_step(c["Hs"], psi, 2e-4)
+    nblk = 8 * 4 * c["nb"]  # one block of two complex wavepackets
+    for _ in range(3):
+        x = [DeviceBuffer(n) for n in 8 * [nblk] + 2 * [41 * nblk] + [1 << 21, 1 << 23, 1 << 25]]
+        for d in x:
+            d.fill_nan()
+            d.free()
+        out, _, _ = c["plan"].propagate(psi, 2e-4, 1, method=evr.SIL, npoly=40, poly_tol=1e-14)
+        assert np.abs(out - ex).max() < 1e-10
+
+
 @pytest.mark.parametrize("method", ["cheby", "sil"])
 def test_field_coupling(evr, sg4_case, method):
     """H_n = H - E_n mu, field constant over each step, a different field per wavepacket."""
