@@ -410,10 +410,9 @@ def keo_grid_run(args):
     e1.record(stream)
     torch.cuda.synchronize()
     ms32 = e0.elapsed_time(e1) / args.steps
-    # algorithmic HBM bytes of the three grid kernels per vector and grid point:
-    # deriv reads psi_G and s, writes D columns; combine reads D columns, D^2
-    # G values and J, writes D; out reads D columns, J and s, writes 1
-    per_point = 8.0 * ((2 + D) + (D + D * D + 1 + D) + (D + 2 + 1))
+    # algorithmic bytes of the grid kernel per vector and grid point: psi_G, s, J,
+    # V and D^2 G values read, one value written
+    per_point = 8.0 * (4 + D * D + 1)
     line = {"workload": "type 10 with G, J, s per grid point, SG4 D=6 L=5 (%d functions, %d grid points), "
                         "%d vectors" % (b.nb_packed, b.sum_nq, nvec),
             "ms_per_hpsi_block": round(ms, 3), "hpsi_per_s_per_vector": round(nvec * 1e3 / ms, 1),
