@@ -29,3 +29,8 @@ int plan_grid_weights(evr_plan *p, const double **gw);
 // Term-concatenated grid order -> the caller's grid order (DP: reference order).
 int plan_grid_to_user(const evr_plan *p, const double *term_grid, double *user);
 }  // namespace evr
+
+// Lays the terms out by given kernel classes: pick[b] (EVR_NCLASSES ints, b <=
+// pick[b]) for the terms whose smallest class is b.  evr_plan_autotune finds
+// such picks by their times; the tests set them.
+extern "C" int evr_plan_set_classes(evr_plan *p, const int *pick);

@@ -202,7 +202,8 @@ struct evr_plan {
   // records, the matrix, factor and coefficient pools, and the work list
   // sorted by class (ht_off; ht_lds[c][lv]: LDS bytes of a workgroup of class
   // c for 1 << lv vectors, ht_items[c]: most pencils of a term).  ht_rest[c]:
-  // terms that stay with the term kernel of class c.
+  // terms that stay with the term kernel of class c, listed with d_order by
+  // apply_classes.
   bool ht = false, ht_hasM = false;
   std::vector<char> ht_on;  // per term: runs in register blocks
   DevBuf<evr::HTerm> d_ht;
@@ -213,8 +214,10 @@ struct evr_plan {
   size_t ht_lds[kHtCaps][4] = {};
   int ht_items[kHtCaps] = {};
   // FP64 basis <-> grid transforms (evr_xform.hip): terms by LDS class, and
-  // those whose reduced grid exceeds a workgroup (x_rest, term kernels)
+  // those whose reduced grid exceeds a workgroup (x_rest, term kernels; listed
+  // by apply_classes)
   bool xt = false;
+  std::vector<char> x_on[2];  // per term: runs in register blocks [grid -> basis, basis -> grid]
   DevBuf<evr::XTerm> d_xt;
   DevBuf<int> d_xorder[2], d_x_rest[2][kNumClasses];  // [grid -> basis, basis -> grid]
   int64_t x_off[2][kXClasses + 1] = {}, x_nrest[2][kNumClasses] = {};
@@ -449,7 +452,10 @@ bool layout_term(const evr_plan *p, evr::TermDev &td, int c, std::vector<evr::St
 
 // Lays out every term for its class p->tclass[t]: slab splits and steps, LDS
 // sizes and flops per class, the per-class work lists (most expensive terms
-// first); uploads the term table, the steps and the lists.
+// first): of all terms, and of those that FP64 H|psi> and the FP64 transforms
+// leave to the term kernels (a term's layout and LDS size are its class's, so
+// no list outlives a change of class); uploads the term table, the steps and
+// the lists.
 int apply_classes(evr_plan *p)
 {
   std::vector<evr::StepDev> steps;
@@ -457,7 +463,11 @@ int apply_classes(evr_plan *p)
     p->lds_bytes64[c] = p->lds_bytes32[c] = 0;
     p->flops_class[c] = 0.0;
     p->nunits[c] = p->nterms_class[c] = 0;
+    p->ht_nrest[c] = p->x_nrest[0][c] = p->x_nrest[1][c] = 0;
     p->d_order[c].release();
+    p->d_ht_rest[c].release();
+    p->d_x_rest[0][c].release();
+    p->d_x_rest[1][c].release();
   }
   std::vector<double> cost(p->nterms);
   for (int64_t t = 0; t < p->nterms; ++t) {
@@ -482,9 +492,19 @@ int apply_classes(evr_plan *p)
     if (ids.empty()) continue;
     std::stable_sort(ids.begin(), ids.end(), [&](int a, int b) { return cost[a] > cost[b]; });
     p->nterms_class[c] = (int64_t)ids.size();
-    while (ids.size() % 8) ids.push_back(-1);
-    p->nunits[c] = (int64_t)ids.size();
-    HIP_TRY(p->d_order[c].upload(ids.data(), ids.size(), p->stream));
+    auto list = [&](const std::vector<char> *skip, DevBuf<int> &buf, int64_t &n) -> int {
+      std::vector<int> l;
+      for (int t : ids)
+        if (!skip || !(*skip)[t]) l.push_back(t);
+      while (l.size() % 8) l.push_back(-1);
+      n = (int64_t)l.size();
+      if (n) HIP_TRY(buf.upload(l.data(), l.size(), p->stream));
+      return EVR_OK;
+    };
+    int rc = list(nullptr, p->d_order[c], p->nunits[c]);
+    if (!rc) rc = list(&p->ht_on, p->d_ht_rest[c], p->ht_nrest[c]);
+    for (int b2g = 0; b2g < 2 && !rc; ++b2g) rc = list(&p->x_on[b2g], p->d_x_rest[b2g][c], p->x_nrest[b2g][c]);
+    if (rc) return rc;
   }
   HIP_TRY(p->d_terms.upload(p->terms.data(), p->terms.size(), p->stream));
   HIP_TRY(p->d_steps.upload(p->steps.data(), p->steps.size(), p->stream));
@@ -1016,7 +1036,7 @@ int build_hterms(evr_plan *p, const HtInput &h)
   // ---- terms
   std::vector<evr::HTerm> ht(p->nterms);
   std::vector<evr::XTerm> xt(p->nterms);
-  std::vector<int> xcap[2], xrest[2][kNumClasses];  // [grid -> basis, basis -> grid]
+  std::vector<int> xcap[2];  // [grid -> basis, basis -> grid]
   xcap[0].assign(p->nterms, -1);
   xcap[1].assign(p->nterms, -1);
   std::vector<evr::HGroup> groups;
@@ -1025,12 +1045,10 @@ int build_hterms(evr_plan *p, const HtInput &h)
   std::vector<int> cap(p->nterms, -1);
   std::vector<double> cost(p->nterms, 0.0);
   std::vector<size_t> words_fix(p->nterms, 0), words_vec(p->nterms, 0);
-  std::vector<int> rest[kNumClasses];
   constexpr size_t kLimit = 160 * 1024 / 8;
   for (int64_t t = 0; t < p->nterms; ++t) {
     const evr::TermDev &td = p->terms[t];
-    const int c = p->tclass[t];
-    if (c < 0) continue;  // streamed
+    if (p->tclass[t] < 0) continue;  // streamed
     evr::HTerm &H = ht[t];
     H.off_nb = td.off_nb;
     H.off_vq = td.off_vq;
@@ -1116,7 +1134,6 @@ int build_hterms(evr_plan *p, const HtInput &h)
         const size_t need = 8 * evr::xform_words(X, b2g);
         for (int k = 0; k < kXClasses; ++k)
           if (need <= (size_t)kXLds[k]) xcap[b2g][t] = k;
-        if (xcap[b2g][t] < 0) xrest[b2g][c].push_back((int)t);
       }
     }
     // pencil mode: the slowest active mode of three functions
@@ -1128,10 +1145,7 @@ int build_hterms(evr_plan *p, const HtInput &h)
         H.nbp = 3;
         std::rotate(act.begin(), act.begin() + k, act.begin() + k + 1);
       }
-    if (p->hasKeo && H.na > evr::kHtModes) {
-      rest[c].push_back((int)t);
-      continue;
-    }
+    if (p->hasKeo && H.na > evr::kHtModes) continue;  // the term kernels
     if (!p->hasKeo) {
       H.na = 0;
       H.nbp = 1;
@@ -1262,10 +1276,7 @@ int build_hterms(evr_plan *p, const HtInput &h)
       wv = std::max(wv, (2 + (size_t)H.nm) * nbt);
       fits = wfix + wv <= kLimit;
     }
-    if (!fits) {
-      rest[c].push_back((int)t);
-      continue;
-    }
+    if (!fits) continue;
     for (int k = 0; k < kHtCaps; ++k)
       if (8 * (wfix + (wv << kHtClasses[k].lv)) <= (size_t)kHtClasses[k].lds) cap[t] = k;
     words_fix[t] = wfix;
@@ -1291,11 +1302,6 @@ int build_hterms(evr_plan *p, const HtInput &h)
     order.insert(order.end(), ids.begin(), ids.end());
   }
   p->ht_off[kHtCaps] = (int64_t)order.size();
-  for (int c = 0; c < kNumClasses; ++c) {
-    while (rest[c].size() % 8) rest[c].push_back(-1);
-    p->ht_nrest[c] = (int64_t)rest[c].size();
-    HIP_TRY(p->d_ht_rest[c].upload(rest[c].data(), rest[c].size(), p->stream));
-  }
   HIP_TRY(p->d_ht.upload(ht.data(), ht.size(), p->stream));
   HIP_TRY(p->d_hg.upload(groups.data(), groups.size(), p->stream));
   HIP_TRY(p->d_hpool.upload(pool.data(), pool.size(), p->stream));
@@ -1317,20 +1323,10 @@ int build_hterms(evr_plan *p, const HtInput &h)
     }
     p->x_off[b2g][kXClasses] = (int64_t)xorder.size();
     HIP_TRY(p->d_xorder[b2g].upload(xorder.data(), xorder.size(), p->stream));
-    for (int c = 0; c < kNumClasses; ++c) {
-      std::vector<int> &r = xrest[b2g][c];
-      while (r.size() % 8) r.push_back(-1);
-      p->x_nrest[b2g][c] = (int64_t)r.size();
-      HIP_TRY(p->d_x_rest[b2g][c].upload(r.data(), r.size(), p->stream));
-    }
+    for (int64_t t = 0; t < p->nterms; ++t) p->x_on[b2g][t] = xcap[b2g][t] >= 0;
   }
   HIP_TRY(p->d_xt.upload(xt.data(), xt.size(), p->stream));
-  if (!keo_ok) {
-    std::fill(cap.begin(), cap.end(), -1);
-    for (int c = 0; c < kNumClasses; ++c) p->ht_nrest[c] = p->nunits[c];
-  }
-  p->ht_on.resize(p->nterms);
-  for (int64_t t = 0; t < p->nterms; ++t) p->ht_on[t] = cap[t] >= 0;
+  for (int64_t t = 0; t < p->nterms; ++t) p->ht_on[t] = keo_ok && cap[t] >= 0;
   p->ht = keo_ok;
   p->xt = true;
   return EVR_OK;
@@ -2357,10 +2353,12 @@ int evr_plan_create(const evr_basis_desc *bd, const evr_op_desc *op, int max_nve
     HIP_TRY(p->d_big.alloc((size_t)(7 + Dk) * p->big_nq * p->big_k));
   }
   {
-    const int rc = apply_classes(p.get());
-    if (rc) return rc;
+    p->ht_on.assign(p->nterms, 0);
+    p->x_on[0] = p->x_on[1] = p->ht_on;
     const int rch = build_hterms(p.get(), HtInput{bw, keo, cC, cA, cF1, sets, D, nlev});
     if (rch) return rch;
+    const int rc = apply_classes(p.get());
+    if (rc) return rc;
     const int rcd = build_dp_terms(p.get(), bw, d1, d2);
     if (rcd) return rcd;
   }
@@ -2776,6 +2774,35 @@ static void recount_flops(evr_plan *p)
   }
 }
 
+// The smallest class that holds each term (-1: streamed, not tuned).
+static std::vector<int> natural_classes(const evr_plan *p)
+{
+  std::vector<int> nat(p->nterms);
+  for (int64_t t = 0; t < p->nterms; ++t) {
+    int c = 0;
+    while (c < kNumClasses && kClasses[c].max_nbt() < p->terms[t].nbt) ++c;
+    nat[t] = c < kNumClasses && p->tclass[t] >= 0 ? c : -1;
+  }
+  return nat;
+}
+
+int evr_plan_set_classes(evr_plan *p, const int *pick)
+{
+  if (!p || !pick) return fail(EVR_ERR_ARG, "NULL argument");
+  for (int b = 0; b < kNumClasses; ++b)
+    if (pick[b] < b || pick[b] >= kNumClasses) return fail(EVR_ERR_ARG, "a bucket needs a class that holds its terms");
+  const std::vector<int> nat = natural_classes(p), old = p->tclass;
+  for (int64_t t = 0; t < p->nterms; ++t)
+    if (nat[t] >= 0) p->tclass[t] = pick[nat[t]];
+  int rc = apply_classes(p);
+  if (rc) {
+    p->tclass = old;
+    (void)apply_classes(p);
+  }
+  recount_flops(p);
+  return rc;
+}
+
 int evr_plan_autotune(evr_plan *p, int nvec, int flags, int reps, int *chosen, double *ms_static,
                       double *ms_tuned)
 {
@@ -2827,12 +2854,7 @@ int evr_plan_autotune(evr_plan *p, int nvec, int flags, int reps, int *chosen, d
   // buckets: terms that share a class under the static rule (smallest class
   // that holds nb_t); each bucket in turn tries the larger classes that hold
   // it, the other buckets keeping their current choice
-  std::vector<int> nat(p->nterms);
-  for (int64_t t = 0; t < p->nterms; ++t) {
-    int c = 0;
-    while (c < kNumClasses && kClasses[c].max_nbt() < p->terms[t].nbt) ++c;
-    nat[t] = c < kNumClasses && p->tclass[t] >= 0 ? c : -1;  // -1: streamed, not tuned
-  }
+  const std::vector<int> nat = natural_classes(p);
   p->tclass = nat;
   int rc = apply_classes(p);
   if (rc) return rc;
