@@ -138,8 +138,7 @@ hipError_t launch_gk_term(const GkArgs<T> &a, int D, int64_t units, int nt, size
     hipLaunchKernelGGL((k_gk_term<T, N>), dim3((unsigned)nblk), dim3(nt), lds, s, a);                \
     break;
   switch (D) {
-    EVR_GK(1) EVR_GK(2) EVR_GK(3) EVR_GK(4) EVR_GK(5) EVR_GK(6)
-    EVR_GK(7) EVR_GK(8) EVR_GK(9) EVR_GK(10) EVR_GK(11) EVR_GK(12)
+    EVR_GK(1) EVR_GK(2) EVR_GK(3) EVR_GK(4) EVR_GK(5) EVR_GK(6) EVR_GK(7) EVR_GK(8) EVR_GK(9)
     default: return hipErrorInvalidValue;
   }
 #undef EVR_GK

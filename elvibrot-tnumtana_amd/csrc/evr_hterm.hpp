@@ -134,6 +134,11 @@ struct GkArgs {
 // spills 164 registers of its 128 (726 us for the H|psi> of D=6 L=5 with 8
 // vectors, 285 us with 2)
 constexpr int kGkPoints = 2;
+// modes the kernel is built for: with ten and more it spills 76 to 179
+// registers and terms of few points run slower than the three passes (8 vectors:
+// D=10 L=5 law 1,1,1,1 721 against 659 us, D=12 L=4 708 against 558 us; D=8 L=5
+// 242 against 307 us)
+constexpr int kGkModes = 9;
 template <typename T>
 hipError_t launch_gk_term(const GkArgs<T> &a, int D, int64_t units, int nt, size_t lds, hipStream_t s);
 

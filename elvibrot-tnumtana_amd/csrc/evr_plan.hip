@@ -1659,8 +1659,12 @@ hipError_t launch_items(int c, const evr::TermParams<double> &prm, int64_t nitem
 }
 
 // psi_G -> the grid form of type 10 on every term (trans: its weighted
-// transpose), one launch per thread count; counts with too few workgroups to
-// fill the device share one.
+// transpose), one launch per thread count.  A launch takes the smaller counts
+// along while its workgroups, all of its own thread count, are at most two
+// rounds of what the CUs hold (D=5 L=5, 2 vectors 58 us, with one round 63 us,
+// with 1024 of any size 78 us), and starts at the first count that a term
+// needs (D=9 L=4, law 1,1,1,1, one vector 50 us, in workgroups of 1024 threads
+// 138 us).
 template <typename T>
 int run_gk_terms(evr_plan *p, int k, int trans, const T *G, T *F)
 {
@@ -1681,8 +1685,13 @@ int run_gk_terms(evr_plan *p, int k, int trans, const T *G, T *F)
   a.sum_nq = p->sum_nq;
   for (int lo = 0; lo < kGkCaps;) {
     int hi = lo + 1;
+    if (p->gk_off[hi] == p->gk_off[lo]) {  // no term of this size
+      lo = hi;
+      continue;
+    }
     size_t lds = p->gk_lds[lo];
-    while (hi < kGkCaps && (p->gk_off[hi + 1] - p->gk_off[lo]) * k <= 4 * (int64_t)p->ncu) {
+    const int64_t rounds = 2 * (int64_t)p->ncu * (1024 / kGkThreads[lo]);
+    while (hi < kGkCaps && (p->gk_off[hi + 1] - p->gk_off[lo]) * k <= rounds) {
       lds = std::max(lds, p->gk_lds[hi]);
       ++hi;
     }
@@ -1836,11 +1845,11 @@ int grid_form_buffers(evr_plan *p)
   if (p->type == 10) {
     std::vector<int> order, cap(p->nterms, -1);
     std::vector<size_t> lds(p->nterms, 0);
-    p->gk_term = true;
-    for (int64_t t = 0; t < p->nterms; ++t) {
+    p->gk_term = D <= evr::kGkModes;
+    for (int64_t t = 0; t < p->nterms && p->gk_term; ++t) {
       const evr::TermDev &td = p->terms[t];
       lds[t] = td.nqt;
-      bool wide = false;  // beyond the kernel's 5-bit digits
+      bool wide = false;  // slots above 32 points: not measured here, they keep the three passes
       for (int d = 0; d < D; ++d) {
         const int nq1 = p->slots[td.slot[d]].nq;
         lds[t] += nq1 * nq1;

@@ -142,3 +142,27 @@ def test_keo_grid_terms(evr, oracle_mod, D, L, law, nvec, herm):
         print("D=%d L=%d law %s hermitian %d: %.3e, FP32 %.3e" % (D, L, law, h, err, err32))
         assert err < 1e-12
         assert err32 < 2e-5
+
+
+@pytest.mark.parametrize("D,L,law,nvec", [
+    (9, 3, (1, 1, 1, 1), 1),    # the most modes of the one-kernel form, terms of 1 to 8 points
+    (10, 2, (1, 1, 2, 1), 3),   # one more: the three passes
+    (5, 4, (1, 2, 2, 2), 2),    # all thread counts in one launch
+    (5, 4, (1, 2, 2, 2), 40),   # a launch per thread count
+    (4, 4, (1, 2, 1, 2), 300)]) # no term of the larger thread counts, more than two rounds
+def test_keo_grid_launches(evr, oracle_mod, D, L, law, nvec):
+    """Grid form with its launches shared and apart, against the oracle."""
+    s = oracle_mod.SG4(D, L, L, *law)
+    b = evr.Basis.sg4(D, L, L, *law)
+    q = s.grid()
+    Gq, J, sq = tabulated_keo(q, 60 + D)
+    V = 0.5 * (q ** 2).sum(1) + 0.05 * q[:, 0] ** 3
+    X = evr.hamiltonian.test_vectors(s.nb_packed, nvec, D)
+    ref = s.oppsi(oracle_mod.Op(10, V=V, Jac=J, s=sq, Gq=Gq), X)
+    plan = evr.Plan(b, type=10, V=V, G0=np.eye(D), max_nvec=nvec)
+    plan.set_keo_grid(Gq, J, sq)
+    err = relerr(plan.TabOpPsi(X), ref)
+    err32 = relerr(plan.TabOpPsi(X, flags=evr.FP32), ref)
+    print("D=%d L=%d law %s, %d vectors: %.3e, FP32 %.3e" % (D, L, law, nvec, err, err32))
+    assert err < 1e-12
+    assert err32 < 2e-5
