@@ -137,19 +137,20 @@ __device__ __forceinline__ void block_top(ctab pool, const HGroup EVR_CONST &G, 
   }
 }
 
-// generic single mode in place: an nb x nb matrix
-__device__ __forceinline__ void generic_in_place(ctab M, int nb, double *io, int s)
+// Rotation of a single mode of any extent nb (stride n1) from x to y, a thread
+// per value: a block of one mode may be all there is, and one lane would then
+// walk its nb x nb matrix alone (12 functions: 9 us a rotation).
+__device__ __forceinline__ void rotate_generic(ctab M, int nb, int n1, int nunit, int lv, const double *x, double *y)
 {
-  double in[kMaxNb];
-#pragma unroll
-  for (int b = 0; b < kMaxNb; ++b)
-    if (b < nb) in[b] = io[b * s];
-  for (int q = 0; q < nb; ++q) {
-    double a = 0.0;
-#pragma unroll
-    for (int b = 0; b < kMaxNb; ++b)
-      if (b < nb) a = fma(M[q * nb + b], in[b], a);
-    io[q * s] = a;
+  const float rn1 = 1.0f / (float)n1, rnb = 1.0f / (float)nb;
+  const int s = n1 << lv;
+  for (int wk = threadIdx.x; wk < nunit; wk += blockDim.x) {
+    const int r = fdiv(wk >> lv, n1, rn1), q = r - fdiv(r, nb, rnb) * nb;
+    const double *in = x + (wk - q * s);
+    const ctab row = M + q * nb;
+    double a = row[0] * in[0];
+    for (int b = 1; b < nb; ++b) a = fma(row[b], in[b * s], a);
+    y[wk] = a;
   }
 }
 
@@ -429,8 +430,10 @@ __global__ __launch_bounds__(1024, 4) void k_hterm(HArgs a)
       sF[i] = i >= lC ? a.coef[td.coef + (i - lC)] : a.fpool[src + (i - base)];
     }
   }
-  // x, the first group rotated on the way in
+  // x, the first group rotated on the way in; groups of any shape rotate from
+  // one of the two tensors to the other, the last of them into sx
   {
+    double *px = a.hasA && (td.ngen & 1) ? sy : sx, *py = a.hasA && (td.ngen & 1) ? sx : sy;
     const int *mp = a.map + td.off_nb;
     const bool rot = a.hasA && ng > 0 && G[0].kind != kHgGeneric;
     if (rot) {
@@ -439,7 +442,7 @@ __global__ __launch_bounds__(1024, 4) void k_hterm(HArgs a)
         const int v = wk & (NV - 1), blk = wk >> lv;
         const int col = v0 + v < a.nvec ? v0 + v : a.nvec - 1;
         const int *m = mp + blk * nb;
-        double *o = sx + ((blk * nb) << lv) + v;
+        double *o = px + ((blk * nb) << lv) + v;
         const int sv = opaque(NV);
         double in[25];
         switch (G[0].kind > kHgSquare ? G[0].kind : G[0].kind + kHgSquare) {
@@ -467,7 +470,7 @@ __global__ __launch_bounds__(1024, 4) void k_hterm(HArgs a)
         const int col = v0 + v < a.nvec ? v0 + v : a.nvec - 1;
         const int pk = mp[e];
         const double xv = X_AT(pk);
-        sx[wk] = pk >= 0 ? xv : 0.0;
+        px[wk] = pk >= 0 ? xv : 0.0;
       }
     }
 #undef X_AT
@@ -475,13 +478,21 @@ __global__ __launch_bounds__(1024, 4) void k_hterm(HArgs a)
     if (a.hasA) {
       for (int g = rot ? 1 : 0; g < ng; ++g) {
         const int nb = G[g].nb, n1 = G[g].n1, nblk = nbt / nb;
+        if (G[g].kind == kHgGeneric) {
+          rotate_generic(a.pool + G[g].mI[0], nb, n1, nunit, lv, px, py);
+          double *const t = px;
+          px = py;
+          py = t;
+          __syncthreads();
+          continue;
+        }
         const float rn1 = 1.0f / (float)n1;
         for (int wk = tid; wk < nblk << lv; wk += nt) {
           const int v = wk & (NV - 1), blk = wk >> lv;
           const int i3 = fdiv(blk, n1, rn1);
-          double *io = sx + ((blk + i3 * n1 * (nb - 1)) << lv) + v;
+          double *io = px + ((blk + i3 * n1 * (nb - 1)) << lv) + v;
           const int s = opaque(n1 << lv);
-          switch (G[g].kind == kHgGeneric ? 0 : (G[g].kind > kHgSquare ? G[g].kind : G[g].kind + kHgSquare)) {
+          switch (G[g].kind > kHgSquare ? G[g].kind : G[g].kind + kHgSquare) {
 #define X(K, B1, N1, B2, N2)                                                                         \
   case K: {                                                                                          \
     double o_[B1 * B2];                                                                              \
@@ -492,7 +503,7 @@ __global__ __launch_bounds__(1024, 4) void k_hterm(HArgs a)
   }
             EVR_HG_SQUARE(X)
 #undef X
-            default: generic_in_place(a.pool + G[g].mI[0], nb, io, s);
+            default: break;
           }
         }
         __syncthreads();
@@ -664,16 +675,25 @@ __global__ __launch_bounds__(1024, 4) void k_hterm(HArgs a)
   {
     const int *rp = a.rowpos + td.off_nb;
     const double w = td.w;
+    double *px = sx, *py = sy;
     if (a.hasA) {
       for (int g = 0; g < ng; ++g) {
         const int nb = G[g].nb, n1 = G[g].n1, nblk = nbt / nb;
+        if (G[g].kind == kHgGeneric) {
+          rotate_generic(a.pool + G[g].mO[0], nb, n1, nunit, lv, py, px);
+          double *const t = px;
+          px = py;
+          py = t;
+          __syncthreads();
+          continue;
+        }
         const float rn1 = 1.0f / (float)n1;
         for (int wk = tid; wk < nblk << lv; wk += nt) {
           const int v = wk & (NV - 1), blk = wk >> lv;
           const int i3 = fdiv(blk, n1, rn1);
-          double *io = sy + ((blk + i3 * n1 * (nb - 1)) << lv) + v;
+          double *io = py + ((blk + i3 * n1 * (nb - 1)) << lv) + v;
           const int s = opaque(n1 << lv);
-          switch (G[g].kind == kHgGeneric ? 0 : (G[g].kind > kHgSquare ? G[g].kind : G[g].kind + kHgSquare)) {
+          switch (G[g].kind > kHgSquare ? G[g].kind : G[g].kind + kHgSquare) {
 #define X(K, B1, N1, B2, N2)                                                                         \
   case K: {                                                                                          \
     double o_[B1 * B2];                                                                              \
@@ -684,7 +704,7 @@ __global__ __launch_bounds__(1024, 4) void k_hterm(HArgs a)
   }
             EVR_HG_SQUARE(X)
 #undef X
-            default: generic_in_place(a.pool + G[g].mO[0], nb, io, s);
+            default: break;
           }
         }
         __syncthreads();
@@ -693,7 +713,7 @@ __global__ __launch_bounds__(1024, 4) void k_hterm(HArgs a)
     for (int wk = tid; wk < nunit; wk += nt) {
       const int v = wk & (NV - 1), e = wk >> lv;
       const int row = rp[e];
-      if (row >= 0 && v0 + v < a.nvec) a.R[(int64_t)row * a.nvec + v0 + v] = w * sy[wk];
+      if (row >= 0 && v0 + v < a.nvec) a.R[(int64_t)row * a.nvec + v0 + v] = w * py[wk];
     }
   }
 }

@@ -53,6 +53,7 @@ struct HTerm {  // sizeof: a multiple of 8
   int wA, wB;              // words per vector of the two V buffers
   int nbO, QO, nO, nOm;    // slabbed V part: functions and points of the outer groups, groups, modes
   int nbI;                 // functions of the inner modes (nbt / nbO)
+  int ngen;                // groups of kind kHgGeneric
   int oB[4], oW[4], onb[4], onq[4];  // matrices and extents of the outer modes
   int coef;                // first coefficient row in the table (hrow_len)
   int nb[kMaxDev], st[kMaxDev];      // functions and stride of the active modes

@@ -1094,6 +1094,7 @@ int build_hterms(evr_plan *p, const HtInput &h)
         G.pw[k] = oO[s] + p->slots[s].nb * p->slots[s].nb - oB[s];
       }
       j += gm1.back() >= 0 ? 2 : 1;
+      H.ngen += G.kind == evr::kHgGeneric;
       groups.push_back(G);
     }
     H.ng = (int)groups.size() - H.g0;

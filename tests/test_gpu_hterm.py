@@ -74,3 +74,77 @@ def test_transforms(evr, oracle_mod, D, L, law, ncol):
     for c in range(ncol):
         ref = s.g2b(Gr[:, c])
         assert np.abs(Y[:, c] - ref).max() / np.abs(ref).max() < TOL64
+
+
+def q_linear(D, rng, symmetric):
+    G0 = np.diag(rng.uniform(1.0, 3.0, D))
+    Ga = rng.uniform(-0.1, 0.1, (D, D, D))
+    if symmetric:  # in all three indices, as the hermitian form needs
+        Ga = sum(Ga.transpose(p) for p in ((0, 1, 2), (0, 2, 1), (1, 0, 2), (1, 2, 0), (2, 0, 1), (2, 1, 0))) / 6.0
+        for i, j, k in np.ndindex(D, D, D):
+            Ga[i, j, k] = Ga[tuple(sorted((i, j, k)))]
+    else:
+        Ga = 0.5 * (Ga + Ga.transpose(1, 0, 2))
+    return G0, Ga.ravel(order="F")
+
+
+@pytest.mark.parametrize("D,L,law,nvec", [
+    (1, 11, (1, 1, 2, 1), 3),                            # one mode, one group of any shape (12 functions)
+    (2, 8, (1, 2, 2, 2), 5),                             # one group of any shape beside a table shape, and none
+    (3, 2, (2, 2, 3, 2), 8), (3, 2, (2, 2, 3, 2), 33),   # three: the classes in one launch, and in several
+    (4, 3, (2, 2, 3, 2), 1), (4, 3, (2, 2, 3, 2), 17),   # four
+    (2, 1, (30, 1, 31, 1), 2)])                          # 30 and 31 functions
+def test_any_shape(evr, oracle_mod, D, L, law, nvec):
+    """Rotations of groups outside the table of shapes, in odd and even number,
+    and launches that several classes share."""
+    rng = np.random.RandomState(D + L + nvec)
+    s = oracle_mod.SG4(D, L, L, *law)
+    b = evr.Basis.sg4(D, L, L, *law)
+    G0, Ga = q_linear(D, rng, False)
+    q = s.grid()
+    V = 0.5 * (q ** 2).sum(axis=1) + 0.1 * q[:, 0] * q[:, -1] ** 2
+    X = np.asfortranarray(rng.randn(b.nb_packed, nvec))
+    ref = s.oppsi(oracle_mod.Op(10, V=V, G0=G0, Ga=Ga), X)
+    e = np.abs(evr.Plan(b, type=10, V=V, G0=G0, Ga=Ga, max_nvec=nvec).TabOpPsi(X) - ref).max() / np.abs(ref).max()
+    print("D=%d L=%d law %s, %d vectors: %.2e" % (D, L, law, nvec, e))
+    assert e < TOL64
+
+
+@pytest.mark.parametrize("D,L,law,nvec", [(3, 4, (1, 2, 2, 2), 3), (5, 3, (1, 2, 1, 2), 8), (4, 2, (2, 1, 3, 1), 2)])
+def test_hermitian(evr, oracle_mod, D, L, law, nvec):
+    """The symmetric form of a q-linear G, (H + H^T) / 2 of the oracle's H."""
+    rng = np.random.RandomState(7 * D + L)
+    s = oracle_mod.SG4(D, L, L, *law)
+    b = evr.Basis.sg4(D, L, L, *law)
+    G0, Ga = q_linear(D, rng, True)
+    q = s.grid()
+    V = 0.5 * (q ** 2).sum(axis=1) + 0.1 * q[:, 0] * q[:, -1] ** 2
+    X = np.asfortranarray(rng.randn(b.nb_packed, nvec))
+    M = s.oppsi(oracle_mod.Op(10, V=V, G0=G0, Ga=Ga), np.asfortranarray(np.eye(b.nb_packed)))
+    ref = 0.5 * (M @ X + M.T @ X)
+    plan = evr.Plan(b, type=10, V=V, G0=G0, Ga=Ga, max_nvec=nvec, hermitian=True)
+    e = np.abs(plan.TabOpPsi(X) - ref).max() / np.abs(ref).max()
+    print("D=%d L=%d law %s, %d vectors: %.2e" % (D, L, law, nvec, e))
+    assert e < TOL64
+
+
+def test_brackets_in_passes(evr, oracle_mod):
+    """Terms whose brackets of all modes do not fit the LDS beside x and y: the
+    kinetic part takes them a few modes at a time."""
+    D, nvec = 4, 2
+    s = oracle_mod.SG4(D, 1, 1, 8, 1, 9, 1)
+    b = evr.Basis.sg4(D, 1, 1, 8, 1, 9, 1)
+    assert 8 * (2 + D) * 8 ** 4 > 160 * 1024 > 8 * (3 * 9 * 8 ** 3 + 2000)
+    rng = np.random.RandomState(5)
+    G0, Ga = q_linear(D, rng, False)
+    q = s.grid()
+    V = 0.5 * (q ** 2).sum(axis=1) + 0.1 * q[:, 0] * q[:, -1] ** 2
+    X = np.asfortranarray(rng.randn(b.nb_packed, nvec))
+    ref = s.oppsi(oracle_mod.Op(10, V=V, G0=G0, Ga=Ga), X)
+    plan = evr.Plan(b, type=10, V=V, G0=G0, Ga=Ga, max_nvec=nvec)
+    plan.set_profiling(True)
+    Y = plan.TabOpPsi(X)
+    assert [n for n, _, _, k in plan.kernel_stats() if k] == ["k_hterm"]
+    e = np.abs(Y - ref).max() / np.abs(ref).max()
+    print("%.2e" % e)
+    assert e < TOL64
