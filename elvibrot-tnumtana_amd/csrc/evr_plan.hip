@@ -1335,8 +1335,13 @@ int build_hterms(evr_plan *p, const HtInput &h)
 
 // The register-block terms of an FP64 H|psi>: one launch per class.  A block
 // of few vectors takes fewer per workgroup (nvec rounded up to a power of
-// two); classes that then agree in it share a launch when their workgroups
-// are too few to fill the device one class at a time.
+// two).  A launch is one chain of a term's phases long however few terms it
+// holds, so a class takes the later ones along, with its own vectors per
+// workgroup, while the workgroups stay within two rounds of what the CUs hold
+// at the shared LDS size (D=4 L=4 law 2,2,3,2, 8 vectors 47 us in one launch,
+// 166 us in four; within four rounds D=4 L=9 with 8 vectors takes 353 us, with
+// two 235 us).  Fewer workgroups than CUs run with all the threads a CU takes
+// (D=6 L=3 law 2,2,3,2, one vector 58 us, with the class's own 74 us).
 int run_hterms(evr_plan *p, int nvec, const double *X, double *R)
 {
   int want = 0;
@@ -1358,24 +1363,33 @@ int run_hterms(evr_plan *p, int nvec, const double *X, double *R)
   a.X = X;
   a.R = R;
   for (int lo = 0; lo < kHtCaps;) {
+    int hi = lo + 1;
+    if (p->ht_off[hi] == p->ht_off[lo]) {  // an empty class
+      lo = hi;
+      continue;
+    }
     a.lv = std::min(kHtClasses[lo].lv, want);
     const int64_t tiles = (nvec + (1 << a.lv) - 1) >> a.lv;
     size_t lds = p->ht_lds[lo][a.lv];
-    int items = p->ht_items[lo] << a.lv, hi = lo + 1, nt = kHtClasses[lo].nt;
-    while (hi < kHtCaps && std::min(kHtClasses[hi].lv, want) == a.lv &&
-           (p->ht_off[hi + 1] - p->ht_off[lo]) * tiles <= 4 * p->ncu) {
-      lds = std::max(lds, p->ht_lds[hi][a.lv]);
-      items = std::max(items, p->ht_items[hi] << a.lv);
-      ++hi;
+    int items = p->ht_items[lo] << a.lv;
+    auto threads = [&](int nt, int most) {  // no more than a thread per item
+      while (nt > 64 && nt / 2 >= most) nt /= 2;
+      return nt;
+    };
+    for (; hi < kHtCaps; ++hi) {
+      const size_t l = std::max(lds, p->ht_lds[hi][a.lv]);
+      const int most = std::max(items, p->ht_items[hi] << a.lv), nt = threads(kHtClasses[lo].nt, most);
+      const int64_t per_cu = std::min<int64_t>(1024 / nt, 160 * kKiB / (int64_t)l);
+      if ((p->ht_off[hi + 1] - p->ht_off[lo]) * tiles > 2 * p->ncu * per_cu) break;
+      lds = l;
+      items = most;
     }
-    const int64_t units = p->ht_off[hi] - p->ht_off[lo];
-    if (units > 0) {
-      while (nt > 64 && nt / 2 >= items) nt /= 2;
-      const int64_t nblk = units * tiles;
-      a.order = (const int EVR_CONST *)(p->d_horder.ptr + p->ht_off[lo]);
-      const hipError_t e = evr::launch_hterm(a, nblk, nt, lds, p->stream);
-      if (e != hipSuccess) return fail(EVR_ERR_HIP, std::string("term kernel: ") + hipGetErrorString(e));
-    }
+    const int64_t nblk = (p->ht_off[hi] - p->ht_off[lo]) * tiles;
+    const int cap = nblk <= p->ncu ? 1024 : (nblk <= 2 * p->ncu ? 512 : 0);
+    const int nt = threads(std::max(kHtClasses[lo].nt, cap), items);
+    a.order = (const int EVR_CONST *)(p->d_horder.ptr + p->ht_off[lo]);
+    const hipError_t e = evr::launch_hterm(a, nblk, nt, lds, p->stream);
+    if (e != hipSuccess) return fail(EVR_ERR_HIP, std::string("term kernel: ") + hipGetErrorString(e));
     lo = hi;
   }
   return EVR_OK;
