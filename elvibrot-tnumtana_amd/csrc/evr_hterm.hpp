@@ -143,13 +143,13 @@ constexpr int kGkModes = 9;
 template <typename T>
 hipError_t launch_gk_term(const GkArgs<T> &a, int D, int64_t units, int nt, size_t lds, hipStream_t s);
 
-// threads and LDS words of a transform workgroup; high r points a wave of the
-// G->B contraction takes at a time
+// most threads and LDS words of a transform workgroup; high r points a wave of
+// the G->B contraction takes at a time
 constexpr int kXThreads = 256;
 constexpr int kXRows = 2;
 size_t xform_words(const XTerm &t, bool b2g);
-// basis -> grid or grid -> basis on n terms x nvec vectors
-hipError_t launch_xform(const XArgs &a, bool b2g, int64_t nterms, size_t lds, hipStream_t s);
+// basis -> grid or grid -> basis on n terms x nvec vectors in workgroups of nt threads (whole waves)
+hipError_t launch_xform(const XArgs &a, bool b2g, int64_t nterms, int nt, size_t lds, hipStream_t s);
 
 // k_hterm on nblk workgroups of nt threads
 hipError_t launch_hterm(const HArgs &a, int64_t nblk, int nt, size_t lds, hipStream_t s);

@@ -222,6 +222,7 @@ struct evr_plan {
   DevBuf<int> d_xorder[2], d_x_rest[2][kNumClasses];  // [grid -> basis, basis -> grid]
   int64_t x_off[2][kXClasses + 1] = {}, x_nrest[2][kNumClasses] = {};
   size_t x_lds[2][kXClasses] = {};
+  int x_pts[2][kXClasses] = {};  // points of the largest term grid
   // work buffers
   DevBuf<double> d_X, d_R, d_psi, d_hpsi, d_G;
   DevBuf<double> d_gw;  // w_t * quadrature weight of every term-grid point (lazy)
@@ -1318,6 +1319,7 @@ int build_hterms(evr_plan *p, const HtInput &h)
         if (xcap[b2g][t] == k) {
           xorder.push_back((int)t);
           p->x_lds[b2g][k] = std::max(p->x_lds[b2g][k], 8 * evr::xform_words(xt[t], b2g));
+          p->x_pts[b2g][k] = std::max(p->x_pts[b2g][k], xt[t].nqt);
         }
       std::stable_sort(xorder.begin() + p->x_off[b2g][k], xorder.end(),
                        [&](int a, int b) { return xt[a].nqt > xt[b].nqt; });
@@ -1425,14 +1427,23 @@ int run_xterms(evr_plan *p, bool b2g, int nvec, const double *X, double *R, doub
   a.gld = p->sum_nq;
   for (int k = 0; k < kXClasses;) {
     // classes too small to fill the device share a launch
-    int hi = k + 1;
+    int hi = k + 1, pts = p->x_pts[b2g][k];
     size_t lds = p->x_lds[b2g][k];
     while (hi < kXClasses && (p->x_off[b2g][hi + 1] - p->x_off[b2g][k]) * nvec <= 8 * (int64_t)p->ncu) {
       lds = std::max(lds, p->x_lds[b2g][hi]);
+      pts = std::max(pts, p->x_pts[b2g][hi]);
       ++hi;
     }
+    // small grids: a wave each, 16 to a CU, as most of a workgroup's threads
+    // would idle (64 vectors G->B: D=10 L=5 law 1,1,1,1 1160 -> 375 us, the term
+    // kernels 781 us; D=12 L=4 law 1,2,1,2, up to 81 points, 691 -> 277 us); from
+    // 64 points on only with workgroups to fill the CUs (D=4 L=4, up to 256
+    // points: 16 vectors 25.6 us, with one wave 27.7 us; 64 vectors 42.7 and
+    // 37.4 us)
+    const int64_t wgs = (p->x_off[b2g][hi] - p->x_off[b2g][k]) * nvec;
+    const int nt = pts <= 64 || (pts <= 256 && wgs > 6 * (int64_t)p->ncu) ? 64 : evr::kXThreads;
     a.order = (const int EVR_CONST *)(p->d_xorder[b2g].ptr + p->x_off[b2g][k]);
-    const hipError_t e = evr::launch_xform(a, b2g, p->x_off[b2g][hi] - p->x_off[b2g][k], lds, p->stream);
+    const hipError_t e = evr::launch_xform(a, b2g, p->x_off[b2g][hi] - p->x_off[b2g][k], nt, lds, p->stream);
     if (e != hipSuccess) return fail(EVR_ERR_HIP, std::string("transform kernel: ") + hipGetErrorString(e));
     k = hi;
   }

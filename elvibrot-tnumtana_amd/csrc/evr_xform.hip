@@ -240,20 +240,20 @@ size_t xform_words(const XTerm &t, bool b2g)
   return (size_t)t.uA + t.uB + t.Pl + Ch + (Ch + t.Rh + Cl + t.Rl + 1) / 2;
 }
 
-hipError_t launch_xform(const XArgs &a, bool b2g, int64_t nterms, size_t lds, hipStream_t s)
+hipError_t launch_xform(const XArgs &a, bool b2g, int64_t nterms, int nt, size_t lds, hipStream_t s)
 {
   const int64_t nblk = nterms * a.nvec;
   if (nblk <= 0) return hipSuccess;
   // the dispatch grid is counted in work-items in 32 bits
-  if (nblk > (int64_t)0xFFFFFFFFu / kXThreads) return hipErrorInvalidConfiguration;
+  if (nblk > (int64_t)0xFFFFFFFFu / nt) return hipErrorInvalidConfiguration;
   if (b2g) {
     (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_b2g), hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)lds);
-    hipLaunchKernelGGL(k_b2g, dim3((unsigned)nblk), dim3(kXThreads), lds, s, a);
+    hipLaunchKernelGGL(k_b2g, dim3((unsigned)nblk), dim3(nt), lds, s, a);
   } else {
     (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_g2b), hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)lds);
-    hipLaunchKernelGGL(k_g2b, dim3((unsigned)nblk), dim3(kXThreads), lds, s, a);
+    hipLaunchKernelGGL(k_g2b, dim3((unsigned)nblk), dim3(nt), lds, s, a);
   }
   return hipGetLastError();
 }

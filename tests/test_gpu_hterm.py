@@ -148,3 +148,23 @@ def test_brackets_in_passes(evr, oracle_mod):
     e = np.abs(Y - ref).max() / np.abs(ref).max()
     print("%.2e" % e)
     assert e < TOL64
+
+
+@pytest.mark.parametrize("D,L,law,ncol", [
+    (10, 2, (1, 1, 1, 1), 5),     # grids of up to 4 points: a wave per term
+    (4, 4, (1, 2, 2, 2), 3),      # up to 256 points: four waves
+    (4, 4, (1, 2, 2, 2), 40)])    # the same in many workgroups: one wave
+def test_transform_workgroups(evr, oracle_mod, D, L, law, ncol):
+    """Transforms in workgroups of one wave and of four."""
+    s = oracle_mod.SG4(D, L, L, *law)
+    b = evr.Basis.sg4(D, L, L, *law)
+    plan = evr.Plan(b, type=0, max_nvec=ncol)
+    rng = np.random.RandomState(D + ncol)
+    X = np.asfortranarray(rng.randn(b.nb_packed, ncol))
+    Gr = np.asfortranarray(rng.randn(b.sum_nq, ncol))
+    G, Y = plan.BasisRep_TO_GridRep_n(X), plan.GridRep_TO_BasisRep_n(Gr)
+    for c in range(ncol):
+        ref = s.b2g(X[:, c])
+        assert np.abs(G[:, c] - ref).max() / np.abs(ref).max() < TOL64
+        ref = s.g2b(Gr[:, c])
+        assert np.abs(Y[:, c] - ref).max() / np.abs(ref).max() < TOL64
