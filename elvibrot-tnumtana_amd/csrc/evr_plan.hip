@@ -213,6 +213,10 @@ struct evr_plan {
   int64_t ht_off[kHtCaps + 1] = {}, ht_nrest[kNumClasses] = {};
   size_t ht_lds[kHtCaps][4] = {};
   int ht_items[kHtCaps] = {};
+  // functions of the terms whose groups all have a shape of the table [0] and
+  // of the others [1]: sums and largest
+  int64_t ht_nb[2] = {};
+  int ht_max[2] = {};
   // FP64 basis <-> grid transforms (evr_xform.hip): terms by LDS class, and
   // those whose reduced grid exceeds a workgroup (x_rest, term kernels; listed
   // by apply_classes)
@@ -1281,6 +1285,8 @@ int build_hterms(evr_plan *p, const HtInput &h)
     if (!fits) continue;
     for (int k = 0; k < kHtCaps; ++k)
       if (8 * (wfix + (wv << kHtClasses[k].lv)) <= (size_t)kHtClasses[k].lds) cap[t] = k;
+    p->ht_nb[H.ngen > 0] += H.nbt;
+    p->ht_max[H.ngen > 0] = std::max(p->ht_max[H.ngen > 0], H.nbt);
     words_fix[t] = wfix;
     words_vec[t] = wv;
     cost[t] = (double)nbt * (4.0 + H.na * H.na + 2.0 * H.ng) * H.QO;
@@ -3005,22 +3011,29 @@ static int ensure_v32(evr_plan *p)
 // against 22.5 ms at 4, 23.3 against 22.8 at 5), at D=12 L=6 the assembled
 // one from 1 vector (2.49 against 2.79 ms).
 //
-// FP64 plans whose terms all run in register blocks (k_hterm) cost, measured
-// at D=9 SG4 L=8 and D=12 SG4 L=6 with 1 to 32 vectors, about 68 ps per term
-// function and vector plus 50 ps per term function and 45 us per call (1.77 /
-// 4.8 / 16.7 / 32.6 ms by the model for 1 / 4 / 16 / 32 vectors at D=9 L=8,
-// measured 1.76 / 4.42 / 16.2 / 32.4); the assembled call adds its term rows
-// to the pool (23.2 ms for one vector, 26.4 ms for 32).  There the
-// sum-factorised path is taken up to 25 vectors (24.6 against 27.6 ms) and up
-// to 7 at D=12 L=6 (1.93 against 2.75 ms); at D=6 SG4 L=5, where both are
-// latency, the assembled one from 1 vector (0.030 against 0.057 ms).
+// An FP64 plan whose terms all run in register blocks (k_hterm) takes, per
+// vector, 68 ps per function of the terms that the shape table covers and 100
+// ps of the others, 20 ps per function for the rows whatever the vectors, and
+// the chain of its largest term: 35 or 70 ns per function.  The assembled call
+// adds its term rows to the pool.  Against 476 timed calls on 34 Smolyak bases
+// (three to twelve modes, seven 1D laws, 1 to 32 vectors; D=9 L=8 and D=12 L=6
+// besides) the choice costs 1.4% over the faster path on average, and none
+// is slower than the choice by the model of the term kernels; without the
+// chain, and with one rate for all shapes, 30 were, up to four times (D=6 L=4
+// law 2,2,3,2, 4 vectors 192 us, assembled 125 us).  At D=9 L=8 the
+// sum-factorised path is taken up to 25 vectors, at D=12 L=6 up to 7, at D=6
+// L=5 the assembled one from 1 vector (0.029 against 0.040 ms).  A one-term
+// plan runs none of these kernels (it streams), and a plan with terms left to
+// the term kernels is priced as if all were.
 static bool matrix_free_cheaper(const evr_plan *p, int nvec, bool fp32)
 {
-  bool ht = p->ht && !fp32;
+  bool ht = p->ht && !fp32 && p->one.empty();
   for (int c = 0; c < kNumClasses; ++c) ht = ht && p->ht_nrest[c] == 0;
   if (ht) {
     const double n = (double)p->sum_nb;
-    return 4.5e-5 + n * (6.8e-11 * nvec + 5.0e-11) < p->asm_bytes64 / 6.0e12 + n * nvec * 4.8e-12 + 2.4e-5;
+    const double t = 3.6e-5 + 2.0e-11 * n + nvec * (6.8e-11 * p->ht_nb[0] + 1.0e-10 * p->ht_nb[1]) +
+                     std::max(3.5e-8 * p->ht_max[0], 7.0e-8 * p->ht_max[1]);
+    return t < p->asm_bytes64 / 6.0e12 + n * nvec * 4.8e-12 + 2.4e-5;
   }
   constexpr double kClassTflops[] = {1.23, 1.82, 2.56, 2.88, 3.83, 5.17, 4.70, 1.99};
   static_assert(sizeof(kClassTflops) / sizeof(double) == kNumClasses, "one rate per term class");

@@ -168,3 +168,22 @@ def test_transform_workgroups(evr, oracle_mod, D, L, law, ncol):
         assert np.abs(G[:, c] - ref).max() / np.abs(ref).max() < TOL64
         ref = s.g2b(Gr[:, c])
         assert np.abs(Y[:, c] - ref).max() / np.abs(ref).max() < TOL64
+
+
+@pytest.mark.parametrize("D,L,law,nvec,kernel", [
+    (6, 7, (1, 2, 2, 2), 1, "k_hterm"),       # 110 us, assembled 169 us
+    (6, 7, (1, 2, 2, 2), 32, "k_apply_asm"),  # 523 us, assembled 226 us
+    (4, 1, (8, 1, 9, 1), 2, "k_apply_asm"),   # five terms, the chain of one: 449 us, assembled 234 us
+    (6, 4, (2, 2, 3, 2), 4, "k_apply_asm")])  # shapes outside the table: 192 us, assembled 125 us
+def test_auto_path(evr, D, L, law, nvec, kernel):
+    """The automatic choice takes the path that is the faster one by far."""
+    b = evr.Basis.sg4(D, L, L, *law)
+    plan = evr.Plan(b, type=10, V=0.5 * (b.grid() ** 2).sum(1), G0=np.eye(D), Ga=np.full(D ** 3, 0.01),
+                    max_nvec=nvec, hermitian=True)
+    plan.assemble(evr.ASM_FP64)
+    X = evr.hamiltonian.test_vectors(b.nb_packed, nvec, 3)
+    ref = plan.TabOpPsi(X, evr.MATRIX_FREE)
+    plan.set_profiling(True)
+    Y = plan.TabOpPsi(X, evr.AUTO_PATH)
+    assert [n for n, _, _, k in plan.kernel_stats() if k] == [kernel]
+    assert np.abs(Y - ref).max() / np.abs(ref).max() < TOL64
