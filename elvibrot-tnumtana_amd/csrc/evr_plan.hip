@@ -6,11 +6,13 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <limits>
 #include <map>
 #include <memory>
 #include <mutex>
 #include <numeric>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "../../include/evr_hip.h"
@@ -864,49 +866,83 @@ struct HtInput {
   const std::vector<std::vector<int>> &sets;   // position -> mode of every coefficient set
   int D;                                       // modes of the coefficients
   int nlev;                                    // slots per mode
+  const std::vector<int> &twin;                // first slot with the same 1D tables
 };
 
-// eigenvectors U (columns) and eigenvalues of the symmetric n x n matrix A by
-// cyclic Jacobi rotations
-void jacobi_eig(int n, std::vector<long double> A, std::vector<long double> &U, std::vector<long double> &lam)
+// eigenvectors U (columns) and eigenvalues of the symmetric n x n matrix A:
+// Householder reflections to tridiagonal form, then QR steps with Wilkinson's
+// shift, each a chase of plane rotations (Golub, Van Loan, Matrix Computations,
+// 8.3).  Cyclic Jacobi sweeps take 3 to 40 times as long here: the coordinate
+// matrix has pairs of opposite eigenvalues and a zero diagonal.
+void sym_eig(int n, std::vector<long double> A, std::vector<long double> &U, std::vector<long double> &lam)
 {
+  using ld = long double;
+  auto a = [&](int i, int j) -> ld & { return A[i + (size_t)n * j]; };
   U.assign((size_t)n * n, 0.0L);
   for (int i = 0; i < n; ++i) U[i + (size_t)n * i] = 1.0L;
-  for (int sweep = 0; sweep < 60; ++sweep) {
-    long double off = 0.0L, all = 0.0L;
-    for (int i = 0; i < n; ++i)
+  std::vector<ld> v(n), w(n);
+  for (int k = 0; k + 2 < n; ++k) {
+    ld tail = 0.0L;
+    for (int i = k + 2; i < n; ++i) tail += a(i, k) * a(i, k);
+    if (tail == 0.0L) continue;
+    const ld x = a(k + 1, k), r = std::sqrt(x * x + tail);
+    ld vv = tail;
+    for (int i = 0; i < n; ++i) v[i] = i > k ? a(i, k) : 0.0L;
+    v[k + 1] = x >= 0.0L ? x + r : x - r;
+    vv += v[k + 1] * v[k + 1];
+    // A <- H A H, U <- U H with H = 1 - 2 v v^T / (v^T v)
+    for (int side = 0; side < 2; ++side)
       for (int j = 0; j < n; ++j) {
-        const long double v = A[i + (size_t)n * j] * A[i + (size_t)n * j];
-        all += v;
-        if (i != j) off += v;
+        ld d = 0.0L;
+        for (int i = k + 1; i < n; ++i) d += v[i] * (side ? a(j, i) : a(i, j));
+        d *= 2.0L / vv;
+        for (int i = k + 1; i < n; ++i) (side ? a(j, i) : a(i, j)) -= d * v[i];
       }
-    if (off <= 1e-38L * all) break;
-    for (int p = 0; p < n; ++p)
-      for (int q = p + 1; q < n; ++q) {
-        const long double apq = A[p + (size_t)n * q];
-        if (apq == 0.0L) continue;
-        const long double th = (A[q + (size_t)n * q] - A[p + (size_t)n * p]) / (2.0L * apq);
-        const long double t = (th >= 0 ? 1.0L : -1.0L) / (std::fabs(th) + std::sqrt(th * th + 1.0L));
-        const long double c = 1.0L / std::sqrt(t * t + 1.0L), s = t * c;
-        for (int k = 0; k < n; ++k) {
-          const long double x = A[k + (size_t)n * p], y = A[k + (size_t)n * q];
-          A[k + (size_t)n * p] = c * x - s * y;
-          A[k + (size_t)n * q] = s * x + c * y;
-        }
-        for (int k = 0; k < n; ++k) {
-          const long double x = A[p + (size_t)n * k], y = A[q + (size_t)n * k];
-          A[p + (size_t)n * k] = c * x - s * y;
-          A[q + (size_t)n * k] = s * x + c * y;
-        }
-        for (int k = 0; k < n; ++k) {
-          const long double x = U[k + (size_t)n * p], y = U[k + (size_t)n * q];
-          U[k + (size_t)n * p] = c * x - s * y;
-          U[k + (size_t)n * q] = s * x + c * y;
-        }
-      }
+    for (int j = 0; j < n; ++j) {
+      ld d = 0.0L;
+      for (int i = k + 1; i < n; ++i) d += v[i] * U[j + (size_t)n * i];
+      d *= 2.0L / vv;
+      for (int i = k + 1; i < n; ++i) U[j + (size_t)n * i] -= d * v[i];
+    }
   }
   lam.resize(n);
-  for (int i = 0; i < n; ++i) lam[i] = A[i + (size_t)n * i];
+  std::vector<ld> e(n, 0.0L);  // e[i]: between i and i + 1
+  for (int i = 0; i < n; ++i) lam[i] = a(i, i);
+  for (int i = 0; i + 1 < n; ++i) e[i] = 0.5L * (a(i, i + 1) + a(i + 1, i));
+  const ld eps = std::numeric_limits<ld>::epsilon();
+  ld all = 0.0L;
+  for (int i = 0; i < n; ++i) all = std::max(all, std::fabs(lam[i]) + std::fabs(e[i]));
+  int hi = n - 1;
+  for (int step = 0; hi > 0 && step < 60 * n; ++step) {
+    if (!(std::fabs(e[hi - 1]) > eps * all)) {
+      e[--hi] = 0.0L;
+      continue;
+    }
+    int lo = hi - 1;
+    while (lo > 0 && std::fabs(e[lo - 1]) > eps * all) --lo;
+    const ld half = 0.5L * (lam[hi - 1] - lam[hi]), b = e[hi - 1], h = std::sqrt(half * half + b * b);
+    const ld mu = lam[hi] - b * b / (half >= 0.0L ? half + h : half - h);
+    ld x = lam[lo] - mu, z = e[lo];
+    for (int k = lo; k < hi; ++k) {
+      const ld r = std::sqrt(x * x + z * z);
+      const ld c = r > 0.0L ? x / r : 1.0L, sn = r > 0.0L ? z / r : 0.0L;
+      if (k > lo) e[k - 1] = r;
+      const ld p = lam[k], q = lam[k + 1], f = e[k];
+      lam[k] = c * c * p + 2.0L * c * sn * f + sn * sn * q;
+      lam[k + 1] = sn * sn * p - 2.0L * c * sn * f + c * c * q;
+      e[k] = c * sn * (q - p) + (c * c - sn * sn) * f;
+      if (k + 1 < hi) {
+        x = e[k];
+        z = sn * e[k + 1];
+        e[k + 1] *= c;
+      }
+      for (int i = 0; i < n; ++i) {
+        const ld u = U[i + (size_t)n * k], t = U[i + (size_t)n * (k + 1)];
+        U[i + (size_t)n * k] = c * u + sn * t;
+        U[i + (size_t)n * (k + 1)] = c * t - sn * u;
+      }
+    }
+  }
 }
 
 // kind of a group of one (nb1 = nq1 = 1) or two modes, kHgGeneric if none
@@ -925,6 +961,14 @@ int hgroup_kind(int nb0, int nq0, int nb1, int nq1)
 int build_hterms(evr_plan *p, const HtInput &h)
 {
   const int D = p->D, Dm = h.D, ns = (int)p->slots.size();
+  std::vector<char> used(ns, 0);  // slots of the terms that run here, and the first of their 1D bases
+  bool any = false;
+  for (int64_t t = 0; t < p->nterms && p->one.empty(); ++t) {  // a one-term plan streams
+    if (p->tclass[t] < 0) continue;
+    any = true;
+    for (int d = 0; d < D; ++d) used[p->terms[t].slot[d]] = used[h.twin[p->terms[t].slot[d]]] = 1;
+  }
+  if (!any) return EVR_OK;
   const bool hasA = p->hasA;
   auto A = [&](int i, int j, int k) { return h.cA[((size_t)i * Dm + j) * Dm + k]; };
   bool keo_ok = true;
@@ -933,8 +977,9 @@ int build_hterms(evr_plan *p, const HtInput &h)
     for (double v : h.cA) amax = std::max(amax, std::fabs(v));
     for (int i = 0; i < Dm; ++i)
       for (int j = 0; j < Dm; ++j) keo_ok = keo_ok && std::fabs(A(j, i, j) - A(i, j, j)) <= 4e-16 * amax;
-    for (const evr::SlotDev &sd : p->slots) {
-      if (sd.nb > evr::kMaxNb) continue;
+    for (int s = 0; s < ns; ++s) {
+      const evr::SlotDev &sd = p->slots[s];
+      if (sd.nb > evr::kMaxNb || h.twin[s] != s) continue;
       const double *Q = h.keo.data() + sd.offK + (size_t)evr::kQ * sd.nb * sd.nb;
       double qmax = 0.0;
       for (int i = 0; i < sd.nb * sd.nb; ++i) qmax = std::max(qmax, std::fabs(Q[i]));
@@ -943,87 +988,100 @@ int build_hterms(evr_plan *p, const HtInput &h)
           keo_ok = keo_ok && std::fabs(Q[i + sd.nb * j] - Q[j + sd.nb * i]) <= 1e-13 * qmax;
     }
   }
-  // ---- per slot: B, W (rotated with a q-linear G) and the rotations, row by
-  // row (a thread's scalar loads take whole rows), and the factor rows
-  // [row][col]{P, T, a_jjj U, R + S} followed by xi
+  // ---- per 1D basis: B, W (rotated with a q-linear G) and the rotations, row
+  // by row (a thread's scalar loads take whole rows); per slot the factor rows
+  // [row][col]{P, T, a_jjj U, R + S} followed by xi.  Modes of one 1D law share
+  // the matrices and the rotated factors.
+  struct Basis1D {
+    int B, W, I, O, P, Q, words;  // offsets in the pool; words of B, W, I, O
+    std::vector<long double> f[4], lam;  // P, T, U, R + S, rotated
+  };
   std::vector<double> pool, fac;
-  std::vector<int> oB(ns), oW(ns), oI(ns), oO(ns), oF(ns), oP(ns), oQ(ns);
+  std::vector<Basis1D> basis(ns);  // at the first slot of every 1D basis
+  std::vector<int> oF(ns, 0);
   const int kTd = p->diagT2 ? evr::kT2 : evr::kT;
+  const bool rotated = hasA && keo_ok;
   for (int s = 0; s < ns; ++s) {
     const evr::SlotDev &sd = p->slots[s];
     const int nb = sd.nb, nq = sd.nq;
-    if (nb > evr::kMaxNb) {  // only streamed terms hold such a slot
-      oB[s] = oW[s] = oI[s] = oO[s] = oF[s] = oP[s] = oQ[s] = 0;
+    if (!used[s]) continue;
+    Basis1D &b1 = basis[h.twin[s]];
+    if (h.twin[s] == s) {
+      const double *B = h.bw.data() + sd.offB, *W = h.bw.data() + sd.offW, *K = h.keo.data() + sd.offK;
+      std::vector<long double> U;
+      b1.lam.assign(nb, 0.0L);
+      auto put = [&](int rows, int cols, auto val) {
+        const int o = (int)pool.size();
+        for (int r = 0; r < rows; ++r)
+          for (int c = 0; c < cols; ++c) pool.push_back((double)val(r, c));
+        while (pool.size() & 1) pool.push_back(0.0);  // 16-byte aligned matrices
+        return o;
+      };
+      auto plainB = [&](int r, int c) { return B[r + (size_t)nq * c]; };
+      auto plainW = [&](int r, int c) { return W[r + (size_t)nb * c]; };
+      if (rotated) {
+        const double *Q = K + (size_t)evr::kQ * nb * nb;
+        std::vector<long double> q((size_t)nb * nb);
+        for (int i = 0; i < nb; ++i)
+          for (int j = 0; j < nb; ++j) q[i + (size_t)nb * j] = 0.5L * ((long double)Q[i + nb * j] + Q[j + nb * i]);
+        sym_eig(nb, q, U, b1.lam);
+        b1.B = put(nq, nb, [&](int r, int c) {
+          long double v = 0.0L;
+          for (int k = 0; k < nb; ++k) v += (long double)B[r + (size_t)nq * k] * U[k + (size_t)nb * c];
+          return v;
+        });
+        b1.W = put(nb, nq, [&](int r, int c) {
+          long double v = 0.0L;
+          for (int k = 0; k < nb; ++k) v += U[k + (size_t)nb * r] * W[k + (size_t)nb * c];
+          return v;
+        });
+        b1.I = put(nb, nb, [&](int r, int c) { return U[c + (size_t)nb * r]; });
+        b1.O = put(nb, nb, [&](int r, int c) { return U[r + (size_t)nb * c]; });
+        b1.words = (int)pool.size() - b1.B;
+        b1.P = put(nq, nb, plainB);
+        b1.Q = put(nb, nq, plainW);
+      } else {
+        b1.P = b1.B = b1.I = b1.O = put(nq, nb, plainB);  // I, O: not used
+        b1.Q = b1.W = put(nb, nq, plainW);
+        b1.words = (int)pool.size() - b1.B;
+      }
+      // U^T F U
+      auto rot = [&](std::vector<long double> F) {
+        if (!rotated) return F;
+        std::vector<long double> t((size_t)nb * nb, 0.0L), o((size_t)nb * nb, 0.0L);
+        for (int j = 0; j < nb; ++j)
+          for (int k = 0; k < nb; ++k)
+            for (int i = 0; i < nb; ++i) t[i + (size_t)nb * j] += F[i + (size_t)nb * k] * U[k + (size_t)nb * j];
+        for (int j = 0; j < nb; ++j)
+          for (int i = 0; i < nb; ++i)
+            for (int k = 0; k < nb; ++k) o[i + (size_t)nb * j] += U[k + (size_t)nb * i] * t[k + (size_t)nb * j];
+        return o;
+      };
+      auto factor = [&](int f) {
+        return std::vector<long double>(K + (size_t)f * nb * nb, K + (size_t)(f + 1) * nb * nb);
+      };
+      b1.f[0] = rot(factor(evr::kP));
+      b1.f[1] = rot(factor(kTd));
+      if (hasA) {
+        std::vector<long double> r = factor(evr::kR), q = factor(evr::kS);
+        for (size_t i = 0; i < r.size(); ++i) r[i] += q[i];
+        b1.f[2] = rot(factor(evr::kU));
+        b1.f[3] = rot(r);
+      } else {
+        b1.f[2].assign((size_t)nb * nb, 0.0L);
+        b1.f[3] = b1.f[2];
+      }
+    } else if (!hasA) {
+      oF[s] = oF[h.twin[s]];
       continue;
     }
-    const double *B = h.bw.data() + sd.offB, *W = h.bw.data() + sd.offW, *K = h.keo.data() + sd.offK;
-    std::vector<long double> U((size_t)nb * nb, 0.0L), lam(nb, 0.0L);
-    for (int i = 0; i < nb; ++i) U[i + (size_t)nb * i] = 1.0L;
-    if (hasA && keo_ok) {
-      const double *Q = K + (size_t)evr::kQ * nb * nb;
-      std::vector<long double> q((size_t)nb * nb);
-      for (int i = 0; i < nb; ++i)
-        for (int j = 0; j < nb; ++j) q[i + (size_t)nb * j] = 0.5L * ((long double)Q[i + nb * j] + Q[j + nb * i]);
-      jacobi_eig(nb, q, U, lam);
-    }
-    auto put = [&](int rows, int cols, auto val) {
-      const int o = (int)pool.size();
-      for (int r = 0; r < rows; ++r)
-        for (int c = 0; c < cols; ++c) pool.push_back((double)val(r, c));
-      while (pool.size() & 1) pool.push_back(0.0);  // 16-byte aligned matrices
-      return o;
-    };
-    oB[s] = put(nq, nb, [&](int r, int c) {
-      long double v = 0.0L;
-      for (int k = 0; k < nb; ++k) v += (long double)B[r + (size_t)nq * k] * U[k + (size_t)nb * c];
-      return v;
-    });
-    oW[s] = put(nb, nq, [&](int r, int c) {
-      long double v = 0.0L;
-      for (int k = 0; k < nb; ++k) v += U[k + (size_t)nb * r] * W[k + (size_t)nb * c];
-      return v;
-    });
-    oI[s] = put(nb, nb, [&](int r, int c) { return U[c + (size_t)nb * r]; });
-    oO[s] = put(nb, nb, [&](int r, int c) { return U[r + (size_t)nb * c]; });
-    oP[s] = oB[s];
-    oQ[s] = oW[s];
-    if (hasA && keo_ok) {
-      oP[s] = put(nq, nb, [&](int r, int c) { return B[r + (size_t)nq * c]; });
-      oQ[s] = put(nb, nq, [&](int r, int c) { return W[r + (size_t)nb * c]; });
-    }
-    // U^T F U
-    auto rot = [&](std::vector<long double> F) {
-      std::vector<long double> t((size_t)nb * nb, 0.0L), o((size_t)nb * nb, 0.0L);
-      for (int i = 0; i < nb; ++i)
-        for (int j = 0; j < nb; ++j)
-          for (int k = 0; k < nb; ++k) t[i + (size_t)nb * j] += F[i + (size_t)nb * k] * U[k + (size_t)nb * j];
-      for (int i = 0; i < nb; ++i)
-        for (int j = 0; j < nb; ++j)
-          for (int k = 0; k < nb; ++k) o[i + (size_t)nb * j] += U[k + (size_t)nb * i] * t[k + (size_t)nb * j];
-      return o;
-    };
-    auto factor = [&](int f) {
-      return std::vector<long double>(K + (size_t)f * nb * nb, K + (size_t)(f + 1) * nb * nb);
-    };
-    std::vector<long double> P = rot(factor(evr::kP)), T = rot(factor(kTd)), Uf, RS;
-    if (hasA) {
-      const int d = s / h.nlev;  // the slot's mode (no compaction with Ga)
-      std::vector<long double> u = factor(evr::kU), r = factor(evr::kR), q = factor(evr::kS);
-      for (size_t i = 0; i < u.size(); ++i) {
-        u[i] *= A(d, d, d);
-        r[i] += q[i];
-      }
-      Uf = rot(u);
-      RS = rot(r);
-    } else {
-      Uf.assign((size_t)nb * nb, 0.0L);
-      RS.assign((size_t)nb * nb, 0.0L);
-    }
+    const int d = hasA ? s / h.nlev : 0;  // the slot's mode (no compaction with Ga)
+    const long double a = hasA ? A(d, d, d) : 0.0L;
     oF[s] = (int)fac.size();
     for (int r = 0; r < nb; ++r)
       for (int c = 0; c < nb; ++c)
-        for (const auto *M : {&P, &T, &Uf, &RS}) fac.push_back((double)(*M)[r + (size_t)nb * c]);
-    for (int c = 0; c < nb; ++c) fac.push_back((double)lam[c]);
+        for (int k = 0; k < 4; ++k) fac.push_back((double)((k == 2 ? a : 1.0L) * b1.f[k][r + (size_t)nb * c]));
+    for (int c = 0; c < nb; ++c) fac.push_back((double)b1.lam[c]);
     if (fac.size() & 1) fac.push_back(0.0);  // 16-byte aligned factor rows
   }
   // ---- coefficients by position of a set
@@ -1046,8 +1104,18 @@ int build_hterms(evr_plan *p, const HtInput &h)
   xcap[1].assign(p->nterms, -1);
   std::vector<evr::HGroup> groups;
   std::vector<double> coef;
-  std::map<std::vector<int>, int> coef_of;
+  struct Hash {
+    size_t operator()(const std::vector<int> &v) const
+    {
+      size_t x = 1469598103934665603ull;
+      for (int i : v) x = (x ^ (size_t)(unsigned)i) * 1099511628211ull;
+      return x;
+    }
+  };
+  std::unordered_map<std::vector<int>, int, Hash> coef_of;
+  std::vector<int> key;
   std::vector<int> cap(p->nterms, -1);
+  groups.reserve((size_t)p->nterms * ((std::min(D, 8) + 1) / 2));
   std::vector<double> cost(p->nterms, 0.0);
   std::vector<size_t> words_fix(p->nterms, 0), words_vec(p->nterms, 0);
   constexpr size_t kLimit = 160 * 1024 / 8;
@@ -1068,37 +1136,34 @@ int build_hterms(evr_plan *p, const HtInput &h)
     }
     // groups over the modes with more than one function
     H.g0 = (int)groups.size();
-    std::vector<int> gm0, gm1;  // modes of every group (gm1: -1 for a single mode)
+    int gm0[evr::kMaxDev], gm1[evr::kMaxDev], ng = 0;  // modes of every group (gm1: -1 for a single mode)
     for (int j = 0; j < td.Dv;) {
       const int d = td.vmode[j];
       const int e = j + 1 < td.Dv ? td.vmode[j + 1] : -1;
       evr::HGroup G{};
-      if (e >= 0 && hgroup_kind(nb[d], nq[d], nb[e], nq[e]) != evr::kHgGeneric) {
-        G.kind = hgroup_kind(nb[d], nq[d], nb[e], nq[e]);
-        gm1.push_back(e);
-      } else {
-        G.kind = hgroup_kind(nb[d], nq[d], 1, 1);
-        gm1.push_back(-1);
-      }
-      gm0.push_back(d);
+      G.kind = e >= 0 ? hgroup_kind(nb[d], nq[d], nb[e], nq[e]) : evr::kHgGeneric;
+      const int modes = G.kind != evr::kHgGeneric ? 2 : 1;
+      if (modes == 1) G.kind = hgroup_kind(nb[d], nq[d], 1, 1);
+      gm0[ng] = d;
+      gm1[ng++] = modes == 2 ? e : -1;
       G.nb = nb[d];
       G.nq = nq[d];
       G.n1 = st[d];
-      for (int k = 0; k < (gm1.back() >= 0 ? 2 : 1); ++k) {
-        const int s = td.slot[k ? e : d];
+      for (int k = 0; k < modes; ++k) {
+        const Basis1D &b1 = basis[h.twin[td.slot[k ? e : d]]];
         if (k) {
           G.nb *= nb[e];
           G.nq *= nq[e];
         }
-        G.mB[k] = oB[s];
-        G.mW[k] = oW[s];
-        G.mI[k] = oI[s];
-        G.mO[k] = oO[s];
-        G.mP[k] = oP[s];
-        G.mQ[k] = oQ[s];
-        G.pw[k] = oO[s] + p->slots[s].nb * p->slots[s].nb - oB[s];
+        G.mB[k] = b1.B;
+        G.mW[k] = b1.W;
+        G.mI[k] = b1.I;
+        G.mO[k] = b1.O;
+        G.mP[k] = b1.P;
+        G.mQ[k] = b1.Q;
+        G.pw[k] = b1.words;
       }
-      j += gm1.back() >= 0 ? 2 : 1;
+      j += modes;
       H.ngen += G.kind == evr::kHgGeneric;
       groups.push_back(G);
     }
@@ -1143,13 +1208,14 @@ int build_hterms(evr_plan *p, const HtInput &h)
       }
     }
     // pencil mode: the slowest active mode of three functions
-    std::vector<int> act(td.amode, td.amode + td.na);
+    int act[evr::kMaxDev];
+    std::copy(td.amode, td.amode + td.na, act);
     H.na = td.na;
     H.nbp = 1;
     for (int k = H.na - 1; k >= 0 && H.nbp == 1; --k)
       if (nb[act[k]] == 3) {
         H.nbp = 3;
-        std::rotate(act.begin(), act.begin() + k, act.begin() + k + 1);
+        std::rotate(act, act + k, act + k + 1);
       }
     if (p->hasKeo && H.na > evr::kHtModes) continue;  // the term kernels
     if (!p->hasKeo) {
@@ -1173,9 +1239,9 @@ int build_hterms(evr_plan *p, const HtInput &h)
     H.fw = fw;
     // coefficient rows of this active list (and its one-function slots)
     {
-      std::vector<int> key{td.cix, H.na, H.nbp};
+      key.assign({td.cix, H.na, H.nbp});
       for (int k = 0; k < H.na; ++k) key.push_back(act[k]);
-      std::vector<char> is_act(D, 0);
+      char is_act[evr::kMaxDev] = {};
       for (int k = 0; k < H.na; ++k) is_act[act[k]] = 1;
       for (int d = 0; d < D; ++d)
         if (!is_act[d]) key.push_back(td.slot[d]);
@@ -1310,31 +1376,32 @@ int build_hterms(evr_plan *p, const HtInput &h)
     order.insert(order.end(), ids.begin(), ids.end());
   }
   p->ht_off[kHtCaps] = (int64_t)order.size();
+  // ---- transforms: terms by LDS class, largest grids first
+  std::vector<int> xorder[2], nqt(p->nterms);
+  for (int64_t t = 0; t < p->nterms; ++t) nqt[t] = p->terms[t].nqt;
+  for (int b2g = 0; b2g < 2; ++b2g) {
+    std::vector<int> &o = xorder[b2g];
+    for (int k = 0; k < kXClasses; ++k) {
+      p->x_off[b2g][k] = (int64_t)o.size();
+      for (int64_t t = 0; t < p->nterms; ++t)
+        if (xcap[b2g][t] == k) {
+          o.push_back((int)t);
+          p->x_lds[b2g][k] = std::max(p->x_lds[b2g][k], 8 * evr::xform_words(xt[t], b2g));
+          p->x_pts[b2g][k] = std::max(p->x_pts[b2g][k], nqt[t]);
+        }
+      std::stable_sort(o.begin() + p->x_off[b2g][k], o.end(), [&](int a, int b) { return nqt[a] > nqt[b]; });
+    }
+    p->x_off[b2g][kXClasses] = (int64_t)o.size();
+    for (int64_t t = 0; t < p->nterms; ++t) p->x_on[b2g][t] = xcap[b2g][t] >= 0;
+  }
   HIP_TRY(p->d_ht.upload(ht.data(), ht.size(), p->stream));
   HIP_TRY(p->d_hg.upload(groups.data(), groups.size(), p->stream));
   HIP_TRY(p->d_hpool.upload(pool.data(), pool.size(), p->stream));
   HIP_TRY(p->d_hfac.upload(fac.data(), fac.size(), p->stream));
   HIP_TRY(p->d_hcoef.upload(coef.data(), coef.size(), p->stream));
   HIP_TRY(p->d_horder.upload(order.data(), order.size(), p->stream));
-  // ---- transforms: terms by LDS class, largest grids first
-  for (int b2g = 0; b2g < 2; ++b2g) {
-    std::vector<int> xorder;
-    for (int k = 0; k < kXClasses; ++k) {
-      p->x_off[b2g][k] = (int64_t)xorder.size();
-      for (int64_t t = 0; t < p->nterms; ++t)
-        if (xcap[b2g][t] == k) {
-          xorder.push_back((int)t);
-          p->x_lds[b2g][k] = std::max(p->x_lds[b2g][k], 8 * evr::xform_words(xt[t], b2g));
-          p->x_pts[b2g][k] = std::max(p->x_pts[b2g][k], xt[t].nqt);
-        }
-      std::stable_sort(xorder.begin() + p->x_off[b2g][k], xorder.end(),
-                       [&](int a, int b) { return xt[a].nqt > xt[b].nqt; });
-    }
-    p->x_off[b2g][kXClasses] = (int64_t)xorder.size();
-    HIP_TRY(p->d_xorder[b2g].upload(xorder.data(), xorder.size(), p->stream));
-    for (int64_t t = 0; t < p->nterms; ++t) p->x_on[b2g][t] = xcap[b2g][t] >= 0;
-  }
   HIP_TRY(p->d_xt.upload(xt.data(), xt.size(), p->stream));
+  for (int b2g = 0; b2g < 2; ++b2g) HIP_TRY(p->d_xorder[b2g].upload(xorder[b2g].data(), xorder[b2g].size(), p->stream));
   for (int64_t t = 0; t < p->nterms; ++t) p->ht_on[t] = keo_ok && cap[t] >= 0;
   p->ht = keo_ok;
   p->xt = true;
@@ -2102,6 +2169,7 @@ int evr_plan_create(const evr_basis_desc *bd, const evr_op_desc *op, int max_nve
   slot_offsets(bd, ox, oB, oD);
   std::vector<double> bw, keo, xs, bwdiag, d1, d2;
   std::vector<char> slot_fold(ns, 0);  // one function with vanishing P, Q, R
+  std::vector<int> twin(ns);           // first slot with the same 1D tables (modes of one 1D law)
   p->slots.resize(ns);
   for (int s = 0; s < ns; ++s) {
     const int nb = bd->nb[s], nq = bd->nq[s];
@@ -2126,6 +2194,22 @@ int evr_plan_create(const evr_basis_desc *bd, const evr_op_desc *op, int max_nve
     sd.offD1 = (int64_t)d1.size();
     d1.insert(d1.end(), bd->D1 + oD[s], bd->D1 + oD[s + 1]);
     d2.insert(d2.end(), bd->D2 + oD[s], bd->D2 + oD[s + 1]);
+    auto same = [&](int t) {
+      auto eq = [](const double *a, const double *b, int64_t n) { return std::memcmp(a, b, sizeof(double) * n) == 0; };
+      return bd->nb[t] == nb && bd->nq[t] == nq && eq(bd->x + ox[t], bd->x + ox[s], nq) &&
+             eq(bd->B + oB[t], bd->B + oB[s], (int64_t)nb * nq) && eq(bd->W + oB[t], bd->W + oB[s], (int64_t)nb * nq) &&
+             eq(bd->D1 + oD[t], bd->D1 + oD[s], (int64_t)nq * nq) && eq(bd->D2 + oD[t], bd->D2 + oD[s], (int64_t)nq * nq);
+    };
+    twin[s] = 0;
+    while (twin[s] < s && (twin[twin[s]] != twin[s] || !same(twin[s]))) ++twin[s];
+    if (twin[s] < s) {
+      const int64_t o = p->slots[twin[s]].offK, n = (int64_t)evr::kNumFactors * nb * nb;
+      sd.offK = (int64_t)keo.size();
+      keo.resize(keo.size() + n);
+      std::copy_n(keo.begin() + o, n, keo.begin() + sd.offK);
+      slot_fold[s] = slot_fold[twin[s]];
+      continue;
+    }
     evr::Slot1D s1;
     s1.nb = nb;
     s1.nq = nq;
@@ -2236,6 +2320,7 @@ int evr_plan_create(const evr_basis_desc *bd, const evr_op_desc *op, int max_nve
       keo[sd.offK + Td] = fTd;
       p->slots.push_back(sd);
       slot_fold.push_back(1);
+      twin.push_back((int)twin.size());
       return (int)p->slots.size() - 1;
     };
     const int unit = add_slot(1.0, 1.0, 0.0);
@@ -2396,7 +2481,7 @@ int evr_plan_create(const evr_basis_desc *bd, const evr_op_desc *op, int max_nve
   {
     p->ht_on.assign(p->nterms, 0);
     p->x_on[0] = p->x_on[1] = p->ht_on;
-    const int rch = build_hterms(p.get(), HtInput{bw, keo, cC, cA, cF1, sets, D, nlev});
+    const int rch = build_hterms(p.get(), HtInput{bw, keo, cC, cA, cF1, sets, D, nlev, twin});
     if (rch) return rch;
     const int rc = apply_classes(p.get());
     if (rc) return rc;
