@@ -208,6 +208,7 @@ struct evr_plan {
   // apply_classes.
   bool ht = false, ht_hasM = false;
   std::vector<char> ht_on;  // per term: runs in register blocks
+  std::vector<double> ht_fV, ht_fK;  // and its operations per vector: V part, the rest
   DevBuf<evr::HTerm> d_ht;
   DevBuf<evr::HGroup> d_hg;
   DevBuf<double> d_hpool, d_hfac, d_hcoef;
@@ -1351,6 +1352,33 @@ int build_hterms(evr_plan *p, const HtInput &h)
     if (!fits) continue;
     for (int k = 0; k < kHtCaps; ++k)
       if (8 * (wfix + (wv << kHtClasses[k].lv)) <= (size_t)kHtClasses[k].lds) cap[t] = k;
+    {  // operations: two for each multiplication and addition of the kernel
+      auto contract = [&](int first, int last, double n, double &f) {  // groups up; f: both ways
+        for (int g = first; g < last; ++g) {
+          const bool two = gm1[g] >= 0;
+          const double b1 = nb[gm0[g]], q1 = nq[gm0[g]], b2 = two ? nb[gm1[g]] : 1, q2 = two ? nq[gm1[g]] : 1;
+          const double blocks = n / (b1 * b2);
+          f += 2.0 * blocks * (q1 * b1 * b2 + (two ? q1 * q2 * b2 : 0.0));      // B
+          f += 2.0 * blocks * ((two ? b2 * q2 * q1 : 0.0) + b1 * q1 * b2);      // W
+          n = blocks * q1 * q2;
+        }
+        return n;
+      };
+      double fV = 0.0, fK = 0.0;
+      const double grid = contract(0, H.ng - H.nO, H.nbI, fV);
+      p->ht_fV[t] = H.QO * (fV + grid + (H.nO ? 4.0 * nbt : 0.0));
+      if (hasA)
+        for (int g = 0; g < H.ng; ++g)
+          fK += 4.0 * nbt * (nb[gm0[g]] + (gm1[g] >= 0 ? nb[gm1[g]] : 0));
+      if (p->hasKeo) {
+        const double na = H.na;
+        double e = 2.0 * na + 2.0;
+        for (int k = 0; k < H.na; ++k) e += 8.0 * H.nb[k] + (hasA ? 2.0 * na : 0.0) + 4.0 + (p->ht_hasM ? 2.0 * H.nb[k] : 0.0);
+        if (p->ht_hasM) e += na * (na - 1.0) * ((hasA ? na - 2.0 : 0.0) + 1.0 + (hasA ? 2.0 : 0.0)) + na;
+        fK += e * nbt;
+      }
+      p->ht_fK[t] = fK;
+    }
     p->ht_nb[H.ngen > 0] += H.nbt;
     p->ht_max[H.ngen > 0] = std::max(p->ht_max[H.ngen > 0], H.nbt);
     words_fix[t] = wfix;
@@ -1567,7 +1595,7 @@ int run_terms(evr_plan *p, int mode, int nvec, const T *X, T *R, T *G, const T *
     if (p->profiling) (void)hipEventRecord(p->ev[2 * c], p->stream);
     hipError_t e = launch_class<T>(c, prm, units, nvec, lds, p->stream);
     if (e != hipSuccess) return fail(EVR_ERR_HIP, std::string("term kernel: ") + hipGetErrorString(e));
-    if (p->profiling) profile_slot(p, c, (blocks ? p->flops_rest[c] : p->flops_class[c]) * nvec);
+    if (p->profiling) profile_slot(p, c, xform ? 0.0 : (blocks ? p->flops_rest[c] : p->flops_class[c]) * nvec);
   }
   if (!p->big.empty()) {
     if (diagKeo) return fail(EVR_ERR_ARG, "the kinetic diagonal of a streamed term is not formed here");
@@ -2480,6 +2508,8 @@ int evr_plan_create(const evr_basis_desc *bd, const evr_op_desc *op, int max_nve
   }
   {
     p->ht_on.assign(p->nterms, 0);
+    p->ht_fV.assign(p->nterms, 0.0);
+    p->ht_fK.assign(p->nterms, 0.0);
     p->x_on[0] = p->x_on[1] = p->ht_on;
     const int rch = build_hterms(p.get(), HtInput{bw, keo, cC, cA, cF1, sets, D, nlev, twin});
     if (rch) return rch;
@@ -2895,7 +2925,7 @@ static void recount_flops(evr_plan *p)
     if (p->tclass[t] < 0) continue;
     const double f = term_flops(p, p->terms[t]);
     p->flops_class[p->tclass[t]] += f;
-    if (p->ht && p->ht_on[t]) p->flops_ht += f;
+    if (p->ht && p->ht_on[t]) p->flops_ht += (p->hasV ? p->ht_fV[t] : 0.0) + p->ht_fK[t];
     else p->flops_rest[p->tclass[t]] += f;
   }
 }

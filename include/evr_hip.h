@@ -317,8 +317,9 @@ int evr_plan_autotune(evr_plan *p, int nvec, int flags, int reps, int *chosen, d
 /* Profiling (no counterpart in the reference, whose analogue is the
  * nb_mult_BTOG/GTOB counters, SYS:120): when on, every term-kernel launch is
  * bracketed by HIP events on the plan stream; evr_plan_kernel_stats returns,
- * per kernel class, the accumulated milliseconds, algorithmic flops and
- * launch count (names: 64 chars each).  Turning it on resets the counters. */
+ * per kernel class, the accumulated milliseconds, algorithmic flops (of H|psi>;
+ * 0 for the FP64 transforms) and launch count (names: 64 chars each).  Turning
+ * it on resets the counters. */
 int evr_plan_set_profiling(evr_plan *p, int on);
 int evr_plan_kernel_stats(evr_plan *p, int max, char *names, double *ms, double *flops,
                           int64_t *launches, int *n);
