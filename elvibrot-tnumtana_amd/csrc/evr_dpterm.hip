@@ -24,8 +24,8 @@
 // 2 vectors: H|psi> 23 us, 77 us with 22 mode-by-mode launches; 17 x 23 x 14, 5
 // vectors 22 us, before 82 us); large ones by the barriers between the steps of
 // the last group, one workgroup of 12 waves per CU (4 x 20 functions, 32
-// vectors: 96 + 355 + 104 us, H|psi> 560 us, 827 us before; its MFMA time alone
-// is 103 us of the 355).  The same with 8 outputs of 64 pencils per wave on
+// vectors: 93 + 362 + 104 us, H|psi> 560 us, 827 us before; its MFMA time alone
+// is 101 us of the 362).  The same with 8 outputs of 64 pencils per wave on
 // scalar coefficients waits for them: 215 + 682 + 123 us.  The matrices in LDS
 // instead of L1 change nothing (351 us), tiles of 4 columns cost 170 us more.
 #include "evr_dpterm.hpp"

@@ -12,11 +12,11 @@
 // back never exist.  The tables of a term are shared by its vectors, which run
 // on one XCD one after the other.
 //
-// Bound: the G table, D^2 values per point and vector from L2, and the 2 D
-// passes over the grid in LDS.  D=6 SG4 L=5, 8 vectors: 191 us in its four
-// launches, the whole H|psi> 258 us against 425 us with the three passes; with
-// the brackets of all modes in LDS at once, and so one to four workgroups per
-// CU, this kernel took 215 us.
+// Bound: the G table, D^2 values per point and vector from L2 (six of seven of
+// its requests hit), and the 2 D passes over the grid in LDS.  D=6 SG4 L=5, 8
+// vectors: 194 us in its three launches, the whole H|psi> 256 us against 425 us
+// with the three passes; with the brackets of all modes in LDS at once, and so
+// one to four workgroups per CU, this kernel took 215 us.
 #include "evr_hterm.hpp"
 
 namespace evr {

@@ -31,16 +31,18 @@
 //  4. y is rotated back and written, weight applied, to the term's rows of R.
 //
 // What bounds it: latency.  A term is small (63 to 2,025 functions carry most
-// of D=9 SG4 L=8), a phase is one wave-length chain of LDS, scalar-cache and
-// FP64 latencies (2,000 to 4,000 cycles; the kinetic bracket 11,000 to 29,000,
-// the gather 13,000), and workgroups hide each other's.  So the phases are few
-// (14 for a six-mode term, where applying one factor at a time between
-// barriers took about 180), the kernel is held to 128 VGPRs for 16 waves per
-// CU, the coefficient rows are staged in LDS beside the factors, and a wave
-// asks for the term's 1D matrices behind the gather, as they are read through
-// the scalar cache.  D=9 SG4 L=8, 32 vectors, type 10 with q-linear G: 31.2 ms
-// against 121.0 ms for the term kernels of evr_term.hip; D=6 L=5, 2 vectors
-// 20.6 against 54.4 us; one vector at D=9 L=8 1.76 against 9.1 ms.
+// of D=9 SG4 L=8) and a phase is one chain of LDS, scalar and FP64 latencies
+// that workgroups hide from each other: the waves wait for 65% of their cycles,
+// and 59% of the vector instructions are indices, addresses and moves of the 56
+// registers that the kernel spills (17 kinetic variants and 16 block shapes
+// share it).  So the phases are few (14 for a six-mode term, where applying one
+// factor at a time between barriers took about 180), the kernel is held to 128
+// VGPRs for 16 waves per CU, the coefficient rows are staged in LDS beside the
+// factors, and a wave asks for the term's 1D matrices behind the gather, as
+// they are read through the scalar cache (1% of its requests miss).  D=9 SG4
+// L=8, 32 vectors, type 10 with q-linear G: 29.0 ms against 121.0 ms for the
+// term kernels of evr_term.hip; D=6 L=5, 2 vectors 15.9 against 54.4 us; one
+// vector at D=9 L=8 1.60 against 9.1 ms.
 #include "evr_hblock.hpp"
 
 namespace evr {

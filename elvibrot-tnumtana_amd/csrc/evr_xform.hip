@@ -16,7 +16,8 @@
 // every term and all combinations of its one-function modes serially.  D=9 SG4
 // L=6, four vectors back (276e6 points, 2.2 GB): 0.65 ms, 3.4 TB/s, against 2.83
 // ms.  A low part of 64 points measured slower (0.218 and 0.665 ms), four r
-// points per wave too (0.73 ms: more LDS, fewer workgroups).
+// points per wave too (0.73 ms: more LDS, fewer workgroups).  Small grids run in
+// workgroups of one wave.
 #include "evr_hblock.hpp"
 
 namespace evr {

@@ -307,10 +307,11 @@ int evr_coupled_oppsi(evr_coupled *c, int nvec, const double *psi, double *hpsi,
  * at the first slower one.  The layout chosen stays with the plan
  * (evr_oppsi, the assembly).  chosen (EVR_NCLASSES ints, or NULL): the class
  * of each bucket; ms_static / ms_tuned: the H|psi> times of the static rule
- * and of the tuned layout.  The classes carry FP32 H|psi>, the assembly and
- * the transforms; FP64 H|psi> runs in register blocks of its own except on
- * terms that those do not take, so its two times agree.  Results are unchanged by the layout (the same
- * arithmetic per term). */
+ * and of the tuned layout.  The classes carry FP32 H|psi> and the assembly;
+ * FP64 H|psi> and the FP64 transforms run in register blocks of their own
+ * except on terms that those do not take (these follow the classes), so the
+ * two FP64 times agree unless a plan has such terms.  Results are unchanged by
+ * the layout (the same arithmetic per term). */
 #define EVR_NCLASSES 8
 int evr_plan_autotune(evr_plan *p, int nvec, int flags, int reps, int *chosen, double *ms_static,
                       double *ms_tuned);
@@ -329,7 +330,10 @@ int evr_plan_kernel_stats(evr_plan *p, int max, char *names, double *ms, double 
  * (OPPSI:701-793) dispatched to sub_TabOpPsi_FOR_SGtype4 (OPSG4:678) for
  * SG4 and to sub_TabOpPsi_WITH_MemGrid_BGG_Hamil10 (OPPSI:1797) for DP.
  * psi, hpsi: nb_packed x nvec column-major.  flags: EVR_FP64 | EVR_FP32,
- * optionally | EVR_DEVICE_PTRS. */
+ * optionally | EVR_DEVICE_PTRS.  Without an assembled operator EVR_FP32 is the
+ * slower precision on SG4 plans (FP64 runs in register blocks, FP32 in the
+ * term kernels: 114 against 30 ms for 32 vectors at D=9 L=8): assemble the FP32
+ * operator before a mixed-precision Davidson or propagation, or stay in FP64. */
 int evr_oppsi(evr_plan *p, int nvec, const double *psi, double *hpsi, int flags);
 
 /* H|psi> with no device allocation (no counterpart in the reference; for
