@@ -882,7 +882,7 @@ void sym_eig(int n, std::vector<long double> A, std::vector<long double> &U, std
   auto a = [&](int i, int j) -> ld & { return A[i + (size_t)n * j]; };
   U.assign((size_t)n * n, 0.0L);
   for (int i = 0; i < n; ++i) U[i + (size_t)n * i] = 1.0L;
-  std::vector<ld> v(n), w(n);
+  std::vector<ld> v(n);
   for (int k = 0; k + 2 < n; ++k) {
     ld tail = 0.0L;
     for (int i = k + 2; i < n; ++i) tail += a(i, k) * a(i, k);
